@@ -1190,12 +1190,12 @@ static int post_stats(cg_ctx *ctx, const unsigned long long *dev_counters, bool 
   return CG_OK;
 }
 
-int cg_posterior(cg_ctx *ctx, const cg_post_args *a)
+// Stages the tables of a posterior call (and `extra`, whose device addresses follow them in dp) in
+// one copy, makes room for the FP64 deferral list, clears the counters and fills p.
+static int post_stage(cg_ctx *ctx, const cg_post_args *a, const std::vector<std::pair<const void *, size_t>> &extra,
+                      std::vector<void *> &dp, cg::PostParams &p)
 {
-  int rc0 = post_validate(ctx, a);
-  if (rc0) return rc0;
   const cg_grid *ref = a->mean[0];
-  DeviceGuard dg(ctx->device);
   const int nyp = ref->nyp, nzp = ref->nzp, cnxp = ref->cnxp;
   const size_t plane = (size_t)cnxp * nyp;
 
@@ -1204,20 +1204,19 @@ int cg_posterior(cg_ctx *ctx, const cg_post_args *a)
   build_plane_tables<float>(a, nzp, t32);
   const bool mixed = a->precision == CG_PREC_MIXED;
   if (mixed) build_plane_tables<double>(a, nzp, t64);
-  std::vector<int> inv(a->invert, a->invert + nzp);
   size_t ninv = 0;
-  for (int v : inv) ninv += (v != 0);
+  for (int k = 0; k < nzp; ++k) ninv += (a->invert[k] != 0);
   std::vector<std::pair<const void *, size_t>> parts = {
       {t32.data(), sizeof(cg::PlaneTab<float>) * nzp},
       {mixed ? (const void *)t64.data() : nullptr, mixed ? sizeof(cg::PlaneTab<double>) * nzp : 0},
-      {inv.data(), sizeof(int) * nzp},
+      {a->invert, sizeof(int) * nzp},
       {a->prior_mode == CG_PRIOR_SEPARABLE ? a->rxy : nullptr, a->prior_mode == CG_PRIOR_SEPARABLE ? sizeof(float) * plane : 0},
       {a->prior_mode == CG_PRIOR_SEPARABLE ? a->rt : nullptr, a->prior_mode == CG_PRIOR_SEPARABLE ? sizeof(float) * nzp : 0},
       {a->err_corr ? nullptr : a->lam2d, a->err_corr ? 0 : sizeof(float) * plane},
   };
+  parts.insert(parts.end(), extra.begin(), extra.end());
   // FP64 deferral list: capacity = inverted cells
   const size_t list_bytes = mixed ? align_up(std::max<size_t>(ninv * plane, 1) * sizeof(unsigned), 256) : 0;
-  std::vector<void *> dp;
   int rc = stage_tables(ctx, parts, dp);
   if (rc) return rc;
   unsigned *list = nullptr;
@@ -1238,7 +1237,7 @@ int cg_posterior(cg_ctx *ctx, const cg_post_args *a)
     }
     list = ctx->list;
   }
-  cg::PostParams p = post_params(a);
+  p = post_params(a);
   p.tab32 = static_cast<const cg::PlaneTab<float> *>(dp[0]);
   p.tab64 = static_cast<const cg::PlaneTab<double> *>(dp[1]);
   p.invert = static_cast<const int *>(dp[2]);
@@ -1250,17 +1249,33 @@ int cg_posterior(cg_ctx *ctx, const cg_post_args *a)
   unsigned long long *cnt = reinterpret_cast<unsigned long long *>(ctx->counters);
   p.list_len = mixed ? cnt : nullptr;
   p.stats = a->stats ? cnt + 8 : nullptr;
-  if (mixed || a->stats) {
-    rc = cg::zero_counters(ctx, cnt, 136);
-    if (rc) return rc;
-  }
-  rc = cg::launch_posterior(ctx, p);
-  if (rc) return rc;
-  for (int g = 0; g < 6; ++g) {  // the covariance grids now hold posterior covariance spectra
+  if (mixed || a->stats) rc = cg::zero_counters(ctx, cnt, 136);
+  return rc;
+}
+
+// The covariance grids of a finished posterior hold posterior covariance spectra.
+static void post_mark(const cg_post_args *a)
+{
+  for (int g = 0; g < 6; ++g) {
     a->cov[g]->transformed = 1;
     a->cov[g]->cubetype = CG_CT_COVARIANCE;
   }
-  if (a->stats) return post_stats(ctx, cnt, mixed, a->stats);
+}
+
+int cg_posterior(cg_ctx *ctx, const cg_post_args *a)
+{
+  int rc0 = post_validate(ctx, a);
+  if (rc0) return rc0;
+  DeviceGuard dg(ctx->device);
+  std::vector<void *> dp;
+  cg::PostParams p;
+  int rc = post_stage(ctx, a, {}, dp, p);
+  if (rc) return rc;
+  rc = cg::launch_posterior(ctx, p);
+  if (rc) return rc;
+  post_mark(a);
+  if (a->stats)
+    return post_stats(ctx, reinterpret_cast<unsigned long long *>(ctx->counters), a->precision == CG_PREC_MIXED, a->stats);
   return CG_OK;
 }
 
@@ -1338,6 +1353,20 @@ int cg_posterior_noalloc(cg_ctx *ctx, const cg_post_args *a)
 }
 
 // ---------------------------------------------------------------------------- simulation
+// Colouring parameters of a grid geometry and its six covariance grids.
+static cg::ColourParams colour_params(const cg_grid *ref, cg_grid *const *cov)
+{
+  cg::ColourParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.csize = (long)ref->csize;
+  p.cnxp = ref->cnxp;
+  p.nyp = ref->nyp;
+  p.nzp = ref->nzp;
+  cg::colour_dims(p);
+  for (int g = 0; g < 6; ++g) p.cov[g] = reinterpret_cast<const float2 *>(cov[g]->d);
+  return p;
+}
+
 // One realisation (next null), or realisations r and r + 1 of one posterior (next: the second's
 // output grids), coloured in one fused launch where the length has one, else one at a time.
 static int simulate_impl(cg_ctx *ctx, const cg_sim_args *a, cg_grid *const *next)
@@ -1378,14 +1407,7 @@ static int simulate_impl(cg_ctx *ctx, const cg_sim_args *a, cg_grid *const *next
     }
   }
   DeviceGuard dg(ctx->device);
-  cg::ColourParams p;
-  std::memset(&p, 0, sizeof(p));
-  p.csize = (long)ref->csize;
-  p.cnxp = ref->cnxp;
-  p.nyp = ref->nyp;
-  p.nzp = ref->nzp;
-  cg::colour_dims(p);
-  for (int g = 0; g < 6; ++g) p.cov[g] = reinterpret_cast<const float2 *>(a->cov[g]->d);
+  cg::ColourParams p = colour_params(ref, a->cov);
   for (int g = 0; g < 3; ++g) p.out[g] = reinterpret_cast<float2 *>(a->out[g]->d);
   for (int g = 0; g < 3; ++g)
     p.mean[g] = spectral == 1 && a->mean[g] ? reinterpret_cast<const float2 *>(a->mean[g]->d) : nullptr;
@@ -1478,6 +1500,241 @@ int cg_simulate_pair(cg_ctx *ctx, const cg_sim_args *a, cg_grid *next_out[3])
   return simulate_impl(ctx, a, next_out);
 }
 
+// ---------------------------------------------------------------------------- passes over several grids
+// The FFT passes of several grids of one geometry in shared launches (descriptor lists), the same
+// kernels and tile variants as grid by grid, so the same bits.  A small grid's pass does not fill
+// the device (64 x 64 x 128 padded to 84 x 84 x 180: 945 workgroups of one wavefront, 9 us for
+// 2 us of traffic), and a request is dozens of them: with 3 angles and a realisation 39 launches
+// and 313 us grid by grid, 13 launches and 179 us in lists.
+}  // extern "C"
+
+namespace {
+
+// Bytes of the grids one launch covers.  Two grids to a launch still gain (200 x 256 x 216, 45 MB
+// each, 5 angles: 909 -> 818 us per inversion; 147 x 256 x 224, 34 MB: 666 -> 604), a launch of
+// one does not (224 x 280 x 200, 51 MB: 1.96 ms grid by grid, 1.99 ms through lists).
+constexpr size_t kListBytes = (size_t)96 << 20;
+
+struct GridPasses {
+  const cg::FixedEntry *x = nullptr, *y = nullptr, *z = nullptr;
+  const cg_grid *ref = nullptr;
+  unsigned chunk = 1;  // grids per launch
+  std::vector<std::vector<char>> blobs;  // descriptors, staged by the caller
+  struct List {
+    int axis, dir, add, n, variant;
+    unsigned blocks;
+    size_t blob;
+  };
+  std::vector<List> lists;
+  const std::vector<void *> *dev = nullptr;  // device addresses of the blobs from dev0 on
+  size_t dev0 = 0;
+
+  // Whether every axis has a compiled plan and a launch holds two grids or more.
+  bool plan(cg_ctx *ctx, const cg_grid *g)
+  {
+    ref = g;
+    if (ctx->fft_engine != CG_FFT_AUTO) return false;
+    const bool even = g->nxp % 2 == 0;
+    x = cg::fixed_find(even ? cg::FIX_XE : cg::FIX_XO, even ? g->nxp / 2 : g->nxp);
+    if (g->nyp > 1) y = cg::fixed_find(cg::FIX_STRIDED, g->nyp);
+    if (g->nzp > 1) z = cg::fixed_find(cg::FIX_STRIDED, g->nzp);
+    const size_t bytes = g->rsize * sizeof(float);
+    chunk = (unsigned)std::min<size_t>(16, kListBytes / bytes);
+    return chunk > 1 && x && (g->nyp == 1 || y) && (g->nzp == 1 || z) && g->csize < (1ul << 27);
+  }
+
+  // axis 0: x (src null: inverse, in place); 1: y; 2: z.  Adds the lists of n grids in chunks and
+  // returns the first list's index; `passes` below runs them.
+  template <class T>
+  void push(int axis, int dir, int add, int variant, const std::vector<T> &items, unsigned blocks)
+  {
+    std::vector<char> b(sizeof(T) * items.size());
+    std::memcpy(b.data(), items.data(), b.size());
+    lists.push_back({axis, dir, add, (int)items.size(), variant, blocks, blobs.size()});
+    blobs.push_back(std::move(b));
+  }
+  void add_x(cg_ctx *ctx, int forward, const float *const *src, float *const *dst, const float *const *add,
+             const float *scale, int n)
+  {
+    const long rows = (long)ref->nyp * ref->nzp;
+    const int v = cg::fixed_variant(ctx, x, rows, forward, add != nullptr);
+    const unsigned nb = (unsigned)((rows + x->tile[v] - 1) / x->tile[v]);
+    std::vector<cg::XArgs> it;
+    for (int i = 0; i < n; ++i)
+      it.push_back({forward ? src[i] : nullptr, dst[i], add ? add[i] : nullptr, rows, nb * (unsigned)i, scale[i]});
+    push(0, forward ? -1 : +1, add != nullptr, v, it, nb * (unsigned)n);
+  }
+  void add_s(cg_ctx *ctx, int axis, int dir, float *const *d, int n)
+  {
+    const cg::FixedEntry *e = axis == 1 ? y : z;
+    if (!e) return;
+    const long cn = ref->cnxp, plane = cn * ref->nyp;
+    const long S = axis == 1 ? cn : plane, inner = S, OS = axis == 1 ? plane : 0;
+    const long ncols = axis == 1 ? cn * ref->nzp : plane;
+    const int v = cg::fixed_variant(ctx, e, S, inner, ncols);
+    const unsigned nb = (unsigned)((ncols + e->tile[v] - 1) / e->tile[v]);
+    std::vector<cg::StridedArgs> it;
+    for (int i = 0; i < n; ++i)
+      it.push_back({reinterpret_cast<float2 *>(d[i]), S, OS, (unsigned)inner, (unsigned)ncols, nb * (unsigned)i, 1.0f});
+    push(axis, dir, 0, v, it, nb * (unsigned)n);
+  }
+  // Forward (x, y, z) or inverse ([z,] y, x) passes of n grids, chunk by chunk.
+  void forward(cg_ctx *ctx, const std::vector<const float *> &src, const std::vector<float *> &dst,
+               const std::vector<float> &scale)
+  {
+    for (size_t i = 0; i < dst.size(); i += chunk) {
+      const int n = (int)std::min<size_t>(chunk, dst.size() - i);
+      add_x(ctx, 1, &src[i], &dst[i], nullptr, &scale[i], n);
+      add_s(ctx, 1, -1, &dst[i], n);
+      add_s(ctx, 2, -1, &dst[i], n);
+    }
+  }
+  void inverse(cg_ctx *ctx, const std::vector<float *> &dst, const std::vector<const float *> &add,
+               const std::vector<float> &scale, bool with_z)
+  {
+    for (size_t i = 0; i < dst.size(); i += chunk) {
+      const int n = (int)std::min<size_t>(chunk, dst.size() - i);
+      if (with_z) add_s(ctx, 2, +1, &dst[i], n);
+      add_s(ctx, 1, +1, &dst[i], n);
+      add_x(ctx, 0, nullptr, &dst[i], add.empty() ? nullptr : &add[i], &scale[i], n);
+    }
+  }
+  int run(cg_ctx *ctx, size_t from, size_t to) const
+  {
+    static const int kclass[3] = {CG_K_FFT_X, CG_K_FFT_Y, CG_K_FFT_Z};
+    for (size_t i = from; i < to; ++i) {
+      const List &l = lists[i];
+      const void *items = (*dev)[dev0 + l.blob];
+      hipEvent_t ev;
+      cg::launch_begin(ctx, kclass[l.axis], &ev);
+      int rc;
+      if (l.axis == 0)
+        rc = cg::fixed_x_list(ctx, x, l.variant, l.dir < 0, l.add, static_cast<const cg::XArgs *>(items), l.n, l.blocks,
+                              ref->nxp);
+      else
+        rc = cg::fixed_strided_list(ctx, l.axis == 1 ? y : z, l.variant, l.dir,
+                                    static_cast<const cg::StridedArgs *>(items), l.n, l.blocks);
+      cg::launch_end(ctx, kclass[l.axis], ev);
+      if (rc) return rc;
+    }
+    return CG_OK;
+  }
+};
+
+}  // namespace
+
+extern "C" {
+
+// cg_invert's drop-in sequence with the passes of its grids in shared launches, every descriptor
+// staged with the posterior's tables in one copy.  Returns 1 where the geometry has no compiled
+// plans or its grids are large, or the arguments are the drop-in calls' to refuse (nothing has run then), else a status.
+static int invert_lists(cg_ctx *ctx, const cg_inversion *v)
+{
+  const cg_post_args &a = v->post;
+  const int nt = a.ntheta;
+  const cg_grid *ref = v->mean_in[0];
+  int n1, n2;
+  GridPasses gp;
+  if (!gp.plan(ctx, ref) || cg::split_z_supported(ref->nxp, ref->nzp, &n1, &n2)) return 1;
+  std::vector<cg_grid *> work(a.mean, a.mean + 3);
+  work.insert(work.end(), a.data, a.data + nt);
+  std::vector<const cg_grid *> in(v->mean_in, v->mean_in + 3);
+  in.insert(in.end(), v->seis_in, v->seis_in + nt);
+  // a shared launch runs every grid's pass at once: no grid may be written for one and read for another
+  std::set<const cg_grid *> distinct(work.begin(), work.end());
+  distinct.insert(in.begin(), in.end());
+  distinct.insert(v->out, v->out + 3 * v->nreal);
+  if (distinct.size() != 2 * work.size() + 3 * (size_t)v->nreal) return 1;
+  std::vector<std::pair<int, int>> before;
+  for (size_t i = 0; i < work.size(); ++i) {
+    before.push_back({work[i]->cubetype, work[i]->transformed});
+    work[i]->cubetype = in[i]->cubetype;
+    work[i]->transformed = 1;
+  }
+  if (post_validate(ctx, &a)) {
+    for (size_t i = 0; i < work.size(); ++i) {
+      work[i]->cubetype = before[i].first;
+      work[i]->transformed = before[i].second;
+    }
+    return 1;
+  }
+  // the scales of grid_fft_forward / grid_fft_inverse
+  const long N = (long)ref->nxp * ref->nyp * ref->nzp;
+  const float s_fwd = 1.0f / sqrtf((float)N), s_inv = float(1.0 / sqrtf(float((size_t)N)));
+  std::vector<const float *> src, means;
+  std::vector<float *> dst, mean;
+  std::vector<float> sf, si;
+  for (size_t i = 0; i < work.size(); ++i) {
+    src.push_back(in[i]->d);
+    dst.push_back(work[i]->d);
+    sf.push_back(in[i]->cubetype == CG_CT_COVARIANCE ? 1.0f : s_fwd);
+  }
+  for (int g = 0; g < 3; ++g) {
+    mean.push_back(a.mean[g]->d);
+    means.push_back(a.mean[g]->d);
+    si.push_back(a.mean[g]->cubetype == CG_CT_COVARIANCE ? float(1.0 / (double)N) : s_inv);
+  }
+  gp.forward(ctx, src, dst, sf);
+  const size_t n_fwd = gp.lists.size();
+  gp.inverse(ctx, mean, {}, si, true);
+  std::vector<size_t> upto = {gp.lists.size()};
+  // realisations: pairs (2m, 2m + 1) as cg_simulate_pair, a last odd one alone; the posterior means
+  // are added in the real domain
+  const long plane = (long)ref->cnxp * ref->nyp;
+  const cg::FixedEntry *one = cg::fixed_colour_entry(ctx, ref->nzp, plane);
+  const cg::FixedEntry *two = cg::fixed_colour2_entry(ctx, ref->nzp, plane);
+  for (int r = 0; r < v->nreal; r += 2) {
+    const int n = r + 1 < v->nreal ? 6 : 3;
+    std::vector<float *> o;
+    std::vector<const float *> add;
+    for (int g = 0; g < n; ++g) {
+      o.push_back(v->out[3 * r + g]->d);
+      add.push_back(means[g % 3]);
+    }
+    gp.inverse(ctx, o, add, std::vector<float>(n, s_inv), !(n == 6 ? two : one));
+    upto.push_back(gp.lists.size());
+  }
+  std::vector<std::pair<const void *, size_t>> extra;
+  for (const auto &b : gp.blobs) extra.push_back({b.data(), b.size()});
+  std::vector<void *> dp;
+  cg::PostParams p;
+  int rc = post_stage(ctx, &a, extra, dp, p);
+  if (rc) return rc;
+  gp.dev = &dp;
+  gp.dev0 = dp.size() - extra.size();
+  rc = gp.run(ctx, 0, n_fwd);
+  if (!rc) rc = cg::launch_posterior(ctx, p);
+  if (rc) return rc;
+  post_mark(&a);
+  rc = gp.run(ctx, n_fwd, upto[0]);
+  if (rc) return rc;
+  for (int g = 0; g < 3; ++g) a.mean[g]->transformed = 0;
+  if (a.stats) {
+    rc = post_stats(ctx, reinterpret_cast<unsigned long long *>(ctx->counters), a.precision == CG_PREC_MIXED, a.stats);
+    if (rc) return rc;
+  }
+  cg::ColourParams cp = colour_params(ref, a.cov);
+  cp.seed = v->seed;
+  for (int r = 0, i = 0; r < v->nreal && !rc; r += 2, ++i) {
+    const bool pair = r + 1 < v->nreal;
+    for (int g = 0; g < 3; ++g) {
+      cp.out[g] = reinterpret_cast<float2 *>(v->out[3 * r + g]->d);
+      cp.out2[g] = pair ? reinterpret_cast<float2 *>(v->out[3 * (r + 1) + g]->d) : nullptr;
+    }
+    cp.stream0 = 3u * (uint32_t)r;
+    cp.stream1 = 3u * (uint32_t)(r + 1);
+    const bool fused = pair ? cg::fixed_colour_zinv2(ctx, cp, cp.nzp, plane, &rc) != 0
+                            : cg::fixed_colour_zinv(ctx, cp, cp.nzp, plane, &rc) != 0;
+    if (!fused) rc = pair ? cg::colour2(ctx, cp) : cg::colour(ctx, cp);
+    if (!rc) rc = gp.run(ctx, upto[i], upto[i + 1]);
+    for (int g = 0; g < (pair ? 6 : 3); ++g) {
+      v->out[3 * r + g]->cubetype = CG_CT_PARAMETER;
+      v->out[3 * r + g]->transformed = rc ? 1 : 0;
+    }
+  }
+  return rc;
+}
+
 // ---------------------------------------------------------------------------- one inversion
 // AVOInversion::computePostMeanResidAndFFTCov (avoinversion.cpp:229-244, 908-1114) and simulate
 // (:1401-1511) for one inversion.  With a compiled split of the z transform (cg_invert.hip) the
@@ -1515,6 +1772,11 @@ int cg_invert(cg_ctx *ctx, const cg_inversion *v)
   const bool split = ctx->fft_engine == CG_FFT_AUTO && !a.want_residual && a.prior_mode == CG_PRIOR_SEPARABLE &&
                      !a.err_corr && a.rxy && a.rt && a.lam2d && cg::split_z_supported(nxp, nzp, &n1, &n2);
   int rc = CG_OK;
+  if (!split) {
+    rc = invert_lists(ctx, v);
+    if (rc <= 0) return rc;
+    rc = CG_OK;
+  }
   std::vector<cg_grid *> work;
   for (int g = 0; g < 3; ++g) work.push_back(a.mean[g]);
   for (int l = 0; l < nt; ++l) work.push_back(a.data[l]);
@@ -1619,14 +1881,7 @@ int cg_invert(cg_ctx *ctx, const cg_inversion *v)
     // the realisations while the means are still in the split layout: the colouring adds them
     // there, and the realisations' inverse passes read nothing else
     if (v->nreal > 0) {
-      cg::ColourParams cp;
-      std::memset(&cp, 0, sizeof(cp));
-      cp.csize = (long)ref->csize;
-      cp.cnxp = cnxp;
-      cp.nyp = nyp;
-      cp.nzp = nzp;
-      cg::colour_dims(cp);
-      for (int g = 0; g < 6; ++g) cp.cov[g] = reinterpret_cast<const float2 *>(a.cov[g]->d);
+      cg::ColourParams cp = colour_params(ref, a.cov);
       cp.seed = v->seed;
       const float2 *ms[3];
       for (int g = 0; g < 3; ++g) ms[g] = reinterpret_cast<const float2 *>(a.mean[g]->d);

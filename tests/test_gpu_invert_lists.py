@@ -1,0 +1,68 @@
+"""cg_invert on small grids runs each FFT pass of its grids in shared launches.  The kernels and
+tile variants are those of the grid-by-grid calls, so the results equal the drop-in calls' bit for
+bit: odd and even lengths, single rows and planes, more grids than one launch holds, an odd and an
+even number of realisations, and the means' work grids being the inputs themselves (which the
+shared launches do not take)."""
+import numpy as np
+import pytest
+
+import crava_amd as C
+import problem as P
+
+pytestmark = pytest.mark.gpu
+
+# (nxp, nyp, nzp), angles, realisations; the fifth has 36 MB grids: two to a launch, five in all
+CASES = [((12, 10, 16), 3, 2), ((9, 7, 15), 5, 1), ((14, 1, 20), 8, 0), ((15, 6, 21), 4, 3), ((250, 180, 200), 2, 1)]
+
+
+def _problem(shape, nt):
+    nxp, nyp, nzp = shape
+    small = nxp * nyp * nzp < 1 << 16
+    p = P.make_problem(max(nxp - 2, 1), max(nyp - 2, 1), max(nzp - 4, 1), nxp=nxp, nyp=nyp if small else 2, nzp=nzp,
+                       angles_deg=tuple(np.linspace(0.0, 40.0, nt)), seed=nxp)
+    if not small:  # the tables of a thin slab, laid over random cubes of the whole size
+        rng = np.random.default_rng(1)
+        p["nyp"], p["ny"] = nyp, nyp - 2
+        for name in ("rxy", "lam2d"):
+            p[name] = np.abs(rng.standard_normal((nyp, nxp // 2 + 1))).astype(np.float32)
+        p["mean_real"] = rng.standard_normal((3, nzp, nyp, nxp), dtype=np.float32)
+        p["seis_real"] = rng.standard_normal((nt, nzp, nyp, nxp), dtype=np.float32)
+    return p
+
+
+def _grids(ctx, p, n, ct, real=None):
+    out = [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    for g, r in zip(out, real if real is not None else ()):
+        g.upload_real(r)
+    return out
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+@pytest.mark.parametrize("in_place", [False, True])
+def test_shared_launches_equal_dropin_calls(ctx, case, in_place):
+    shape, nt, nreal = CASES[case]
+    print("shared launches", shape, nt, nreal, in_place, flush=True)
+    p = _problem(shape, nt)
+    mean_in, seis_in = _grids(ctx, p, 3, C.PARAMETER, p["mean_real"]), _grids(ctx, p, nt, C.DATA, p["seis_real"])
+    mean, data, cov = (_grids(ctx, p, n, t) for n, t in ((3, C.PARAMETER), (nt, C.DATA), (6, C.COVARIANCE)))
+    outs = [_grids(ctx, p, 3, C.PARAMETER) for _ in range(nreal)]
+    for g, s in zip(mean + data, mean_in + seis_in):
+        g.fft_from(s)
+    want_stats = C.posterior(ctx, p, mean, data, cov, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], want_residual=False,
+                             precision=C.PREC_MIXED)
+    for g in mean:
+        g.invFFTInPlace()
+    for r in range(0, nreal, 2):
+        C.simulate(ctx, cov, mean, outs[r], seed=9, realisation=r, next_out=outs[r + 1] if r + 1 < nreal else None)
+    want = [g.download_real() for g in mean] + [g.download_complex() for g in cov] + \
+           [g.download_real() for r in outs for g in r]
+    item = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=9, mean_in=mean_in, seis_in=seis_in,
+                mean=mean_in if in_place else mean, data=data, cov=cov, out=outs)
+    stats = C.invert(ctx, item, stats=True)
+    got = [g.download_real() for g in item["mean"]] + [g.download_complex() for g in cov] + \
+          [g.download_real() for r in outs for g in r]
+    assert stats == want_stats
+    for w, g in zip(want, got):
+        assert np.array_equal(w, g)
+    for g in mean_in + seis_in + mean + data + cov + [g for r in outs for g in r]:
+        g.close()
