@@ -8,6 +8,7 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <functional>
 #include <new>
 
 #include "cg_internal.h"
@@ -38,7 +39,8 @@ struct DeviceGuard {
 
 
 // Pinned staging of small host tables into one device buffer on the context stream.
-int stage_tables(cg_ctx *ctx, const std::vector<std::pair<const void *, size_t>> &parts, std::vector<void *> &dptrs)
+int stage_tables(cg_ctx *ctx, const std::vector<std::pair<const void *, size_t>> &parts, std::vector<void *> &dptrs,
+                 const std::function<void(const std::vector<void *> &)> &placed = nullptr)
 {
   size_t total = 0;
   for (auto &p : parts) total += align_up(p.second, 256);
@@ -64,8 +66,13 @@ int stage_tables(cg_ctx *ctx, const std::vector<std::pair<const void *, size_t>>
   size_t off = 0;
   dptrs.clear();
   for (auto &p : parts) {
-    if (p.second) std::memcpy(h + off, p.first, p.second);
     dptrs.push_back(p.second ? dev + off : nullptr);
+    off += align_up(p.second, 256);
+  }
+  if (placed) placed(dptrs);
+  off = 0;
+  for (auto &p : parts) {
+    if (p.second) std::memcpy(h + off, p.first, p.second);
     off += align_up(p.second, 256);
   }
   hipError_t e = hipMemcpyAsync(dev, h, off ? off : 256, hipMemcpyHostToDevice, ctx->stream);
@@ -1192,8 +1199,11 @@ static int post_stats(cg_ctx *ctx, const unsigned long long *dev_counters, bool 
 
 // Stages the tables of a posterior call (and `extra`, whose device addresses follow them in dp) in
 // one copy, makes room for the FP64 deferral list, clears the counters and fills p.
+// placed, if given, is told the addresses and the index of the first extra part before the copy, so
+// that parts may hold addresses of others.
 static int post_stage(cg_ctx *ctx, const cg_post_args *a, const std::vector<std::pair<const void *, size_t>> &extra,
-                      std::vector<void *> &dp, cg::PostParams &p)
+                      std::vector<void *> &dp, cg::PostParams &p,
+                      const std::function<void(const std::vector<void *> &, size_t)> &placed = nullptr)
 {
   const cg_grid *ref = a->mean[0];
   const int nyp = ref->nyp, nzp = ref->nzp, cnxp = ref->cnxp;
@@ -1217,7 +1227,8 @@ static int post_stage(cg_ctx *ctx, const cg_post_args *a, const std::vector<std:
   parts.insert(parts.end(), extra.begin(), extra.end());
   // FP64 deferral list: capacity = inverted cells
   const size_t list_bytes = mixed ? align_up(std::max<size_t>(ninv * plane, 1) * sizeof(unsigned), 256) : 0;
-  int rc = stage_tables(ctx, parts, dp);
+  int rc = stage_tables(ctx, parts, dp, placed ? [&](const std::vector<void *> &d) { placed(d, 6); }
+                                               : std::function<void(const std::vector<void *> &)>());
   if (rc) return rc;
   unsigned *list = nullptr;
   if (mixed) {
@@ -1515,6 +1526,17 @@ namespace {
 // one does not (224 x 280 x 200, 51 MB: 1.96 ms grid by grid, 1.99 ms through lists).
 constexpr size_t kListBytes = (size_t)96 << 20;
 
+// The band-limited sequence: grids too large for shared launches (the cubes that are batched are
+// smaller, and an inversion of theirs has the same bits alone and in a batch), whose inverted
+// frequencies fill at most these parts of the planes.  Mean and covariance at 224 x 280 x 200, 5
+// angles, by the share of the planes that the band fills (microseconds, all wavenumbers / band):
+// 40% 951 / 579, 56% 958 / 673, 72% 972 / 805, 84% 981 / 989; on a split-z geometry (576 x 576 x 320)
+// 40% 5832 / 4442, 48% 5897 / 4911, and its line crosses near 65%.
+constexpr size_t kBandBytes = kListBytes / 2;
+constexpr double kBandMost = 0.75, kBandMostSplit = 0.62;
+// Bytes of the band planes one launch of it covers.
+constexpr size_t kBandChunk = (size_t)96 << 20;
+
 struct GridPasses {
   const cg::FixedEntry *x = nullptr, *y = nullptr, *z = nullptr;
   const cg_grid *ref = nullptr;
@@ -1624,6 +1646,151 @@ struct GridPasses {
 }  // namespace
 
 extern "C" {
+
+// cg_invert's band-limited sequence (cg_band.h): the posterior of large grids whose inverted planes
+// are few.  Returns 1 where it does not apply (nothing has run then), else a status; the
+// realisations are left to the caller, the means end in the real domain.
+//   (3 + nt) x  z forward (real cube -> band planes), x, y forward
+//   1 x         posterior of the band, covariance of every plane
+//   3 x         y, x inverse of the update, z inverse + prior mean
+// The band planes of an input live in its work grid; the inverse x passes move the three updates
+// into seismic work grids, since the last pass writes the means' own.
+static int invert_band(cg_ctx *ctx, const cg_inversion *v)
+{
+  const cg_post_args &a = v->post;
+  const int nt = a.ntheta;
+  const cg_grid *ref = v->mean_in[0];
+  const int nxp = ref->nxp, nyp = ref->nyp, nzp = ref->nzp, cnxp = ref->cnxp;
+  if (ctx->fft_engine != CG_FFT_AUTO || a.want_residual || a.prior_mode != CG_PRIOR_SEPARABLE || a.err_corr || !a.rxy ||
+      !a.rt || !a.lam2d || !a.invert || (a.precision != CG_PREC_REFERENCE && a.precision != CG_PREC_MIXED))
+    return 1;
+  if (ref->rsize * sizeof(float) <= kBandBytes || ref->csize >= (1ul << 31)) return 1;
+  const cg::FixedEntry *ex = cg::fixed_find(cg::FIX_STRIDED, nxp), *ez = cg::fixed_find(cg::FIX_STRIDED, nzp);
+  const cg::FixedEntry *ey = nyp > 1 ? cg::fixed_find(cg::FIX_STRIDED, nyp) : nullptr;
+  if (!ex || !ez || (nyp > 1 && !ey)) return 1;
+  std::vector<int> kb, at(nzp / 2 + 1, -1);
+  for (int k = 0; k <= nzp / 2; ++k)
+    if (a.invert[k] || a.invert[k ? nzp - k : 0]) {
+      at[k] = (int)kb.size();
+      kb.push_back(k);
+    }
+  const size_t nb = kb.size(), plane = (size_t)cnxp * nyp, cells = nb * plane * 2;
+  // where the band is worth it, and three updates fit the seismic work grids
+  int n1, n2;
+  const double most = cg::split_z_supported(nxp, nzp, &n1, &n2) ? kBandMostSplit : kBandMost;
+  if (nb == 0 || 2.0 * nb > most * nzp) return 1;
+  const size_t per = ref->csize / cells;
+  if (per * nt < 3) return 1;
+  std::vector<cg_grid *> work(a.mean, a.mean + 3);
+  work.insert(work.end(), a.data, a.data + nt);
+  std::vector<const cg_grid *> in(v->mean_in, v->mean_in + 3);
+  in.insert(in.end(), v->seis_in, v->seis_in + nt);
+  std::set<const cg_grid *> distinct(work.begin(), work.end());
+  distinct.insert(in.begin(), in.end());
+  distinct.insert(a.cov, a.cov + 6);
+  if (distinct.size() != 2 * work.size() + 6) return 1;
+  std::vector<std::pair<int, int>> before;
+  for (size_t i = 0; i < work.size(); ++i) {
+    before.push_back({work[i]->cubetype, work[i]->transformed});
+    work[i]->cubetype = in[i]->cubetype;
+    work[i]->transformed = 1;
+  }
+  if (post_validate(ctx, &a)) {  // the drop-in calls refuse it
+    for (size_t i = 0; i < work.size(); ++i) {
+      work[i]->cubetype = before[i].first;
+      work[i]->transformed = before[i].second;
+    }
+    return 1;
+  }
+  // descriptors: one per grid and pass, the launches take runs of `chunk` of them
+  const long N = (long)nxp * nyp * nzp;
+  const float s_fwd = 1.0f / sqrtf((float)N), s_inv = float(1.0 / sqrtf(float((size_t)N)));
+  const int n = 3 + nt;
+  const int chunk = (int)std::min<size_t>(16, std::max<size_t>(1, kBandChunk / (cells * sizeof(float2))));
+  const unsigned zb = (unsigned)((plane + ez->bz_tile - 1) / ez->bz_tile);
+  const unsigned xb = (unsigned)((nb * nyp + ex->bx_rows - 1) / ex->bx_rows);
+  const long ncols_y = (long)(2 * cnxp) * (long)nb;
+  const int vy = ey ? cg::fixed_variant(ctx, ey, 2 * cnxp, 2 * cnxp, ncols_y) : 0;
+  const unsigned yb = ey ? (unsigned)((ncols_y + ey->tile[vy] - 1) / ey->tile[vy]) : 0;
+  std::vector<cg::BandArgs> zf, xf, xi, zi;
+  std::vector<cg::StridedArgs> yf, yi;
+  for (int i = 0; i < n + 3; ++i) {  // the inputs, then the three updates
+    const bool fwd = i < n;
+    const int g = fwd ? i : i - n, s = (fwd ? i : g) % chunk;
+    cg_grid *w = work[g];
+    cg::BandArgs b;
+    std::memset(&b, 0, sizeof(b));
+    b.rows = (long)(nb * nyp);
+    b.nb = (unsigned)nb;
+    b.ncols = (unsigned)plane;
+    b.cnxp = (unsigned)cnxp;
+    b.nxp = nxp;
+    b.real = in[g]->d;
+    b.out = w->d;
+    b.band = reinterpret_cast<float2 *>(w->d);
+    b.band_out = fwd ? b.band : reinterpret_cast<float2 *>(a.data[g % nt]->d) + (size_t)(g / nt) * cells;
+    b.block0 = xb * (unsigned)s;
+    (fwd ? xf : xi).push_back(b);
+    const cg::StridedArgs y{b.band, 2 * cnxp, (long)(2 * plane), (unsigned)(2 * cnxp), (unsigned)ncols_y, yb * (unsigned)s, 1.0f};
+    (fwd ? yf : yi).push_back(y);
+    if (!fwd) b.band = b.band_out;
+    b.block0 = zb * (unsigned)s;
+    b.scale = in[g]->cubetype == CG_CT_COVARIANCE ? (fwd ? 1.0f : float(1.0 / (double)N)) : (fwd ? s_fwd : s_inv);
+    (fwd ? zf : zi).push_back(b);
+  }
+  // the frequency tables and descriptors are staged with the posterior's tables; the descriptors get
+  // the tables' addresses once the layout is known
+  std::vector<std::pair<const void *, size_t>> extra = {{kb.data(), sizeof(int) * nb}, {at.data(), sizeof(int) * at.size()}};
+  for (const auto *l : {&zf, &xf, &xi, &zi}) extra.push_back({l->data(), sizeof(cg::BandArgs) * l->size()});
+  for (const auto *l : {&yf, &yi}) extra.push_back({l->data(), sizeof(cg::StridedArgs) * l->size()});
+  std::vector<void *> dp;
+  cg::PostBandArgs pb;
+  int rc = post_stage(ctx, &a, extra, dp, pb.p, [&](const std::vector<void *> &d, size_t first) {
+    for (auto *l : {&zf, &xf, &xi, &zi})
+      for (auto &b : *l) {
+        b.kb = static_cast<const int *>(d[first]);
+        b.at = static_cast<const int *>(d[first + 1]);
+      }
+  });
+  if (rc) return rc;
+  const size_t e0 = dp.size() - extra.size();
+  pb.at = static_cast<const int *>(dp[e0 + 1]);
+  pb.by_cnxp = cg::make_fastdiv((uint32_t)cnxp);
+  pb.rnxp = 2u * (unsigned)cnxp;
+  const cg::BandArgs *dz = static_cast<const cg::BandArgs *>(dp[e0 + 2]), *dx = static_cast<const cg::BandArgs *>(dp[e0 + 3]),
+                     *dxi = static_cast<const cg::BandArgs *>(dp[e0 + 4]), *dzi = static_cast<const cg::BandArgs *>(dp[e0 + 5]);
+  const cg::StridedArgs *dy = static_cast<const cg::StridedArgs *>(dp[e0 + 6]), *dyi = static_cast<const cg::StridedArgs *>(dp[e0 + 7]);
+  const float2 *twx = cg::twiddle_table(ctx, nxp), *twz = cg::twiddle_table(ctx, nzp);
+  if (!twx || !twz) return CG_ENOMEM;
+  auto timed = [&](int kclass, auto f) {
+    hipEvent_t ev;
+    if (rc) return;
+    cg::launch_begin(ctx, kclass, &ev);
+    rc = f();
+    cg::launch_end(ctx, kclass, ev);
+  };
+  for (int i = 0; i < n; i += chunk) {
+    const int c = std::min(chunk, n - i);
+    timed(CG_K_FFT_Z, [&] { return ez->bz(ctx, -1, dz + i, c, zb * (unsigned)c, twz); });
+    timed(CG_K_FFT_X, [&] { return ex->bx(ctx, -1, dx + i, c, xb * (unsigned)c, twx); });
+    if (ey) timed(CG_K_FFT_Y, [&] { return cg::fixed_strided_list(ctx, ey, vy, -1, dy + i, c, yb * (unsigned)c); });
+  }
+  if (rc) return rc;
+  rc = cg::launch_posterior_band(ctx, pb);
+  if (rc) return rc;
+  post_mark(&a);
+  for (int i = 0; i < 3; i += chunk) {
+    const int c = std::min(chunk, 3 - i);
+    if (ey) timed(CG_K_FFT_Y, [&] { return cg::fixed_strided_list(ctx, ey, vy, +1, dyi + i, c, yb * (unsigned)c); });
+    timed(CG_K_FFT_X, [&] { return ex->bx(ctx, +1, dxi + i, c, xb * (unsigned)c, twx); });
+    timed(CG_K_FFT_Z, [&] { return ez->bz(ctx, +1, dzi + i, c, zb * (unsigned)c, twz); });
+  }
+  if (rc) return rc;
+  for (int g = 0; g < 3; ++g) a.mean[g]->transformed = 0;
+  if (a.stats)
+    rc = post_stats(ctx, reinterpret_cast<unsigned long long *>(ctx->counters), a.precision == CG_PREC_MIXED, a.stats);
+  return rc;
+}
 
 // cg_invert's drop-in sequence with the passes of its grids in shared launches, every descriptor
 // staged with the posterior's tables in one copy.  Returns 1 where the geometry has no compiled
@@ -1771,17 +1938,21 @@ int cg_invert(cg_ctx *ctx, const cg_inversion *v)
   int n1 = 0, n2 = 0;
   const bool split = ctx->fft_engine == CG_FFT_AUTO && !a.want_residual && a.prior_mode == CG_PRIOR_SEPARABLE &&
                      !a.err_corr && a.rxy && a.rt && a.lam2d && cg::split_z_supported(nxp, nzp, &n1, &n2);
-  int rc = CG_OK;
-  if (!split) {
+  int rc = invert_band(ctx, v);
+  const bool band = rc <= 0;
+  if (rc < 0) return rc;
+  if (!band && !split) {
     rc = invert_lists(ctx, v);
     if (rc <= 0) return rc;
-    rc = CG_OK;
   }
+  rc = CG_OK;
   std::vector<cg_grid *> work;
   for (int g = 0; g < 3; ++g) work.push_back(a.mean[g]);
   for (int l = 0; l < nt; ++l) work.push_back(a.data[l]);
   auto input = [&](int i) { return i < 3 ? v->mean_in[i] : v->seis_in[i - 3]; };
-  if (!split) {
+  if (band) {
+    // the means are in the real domain
+  } else if (!split) {
     for (int i = 0; i < 3 + nt && !rc; ++i) {
       work[i]->cubetype = input(i)->cubetype;
       rc = cg::grid_fft_forward(work[i], input(i)->d);
@@ -1917,7 +2088,7 @@ int cg_invert(cg_ctx *ctx, const cg_inversion *v)
     }
     if (!rc && a.stats) rc = post_stats(ctx, cnt, mixed, a.stats);
   }
-  if (rc || split) return rc;
+  if (rc || (split && !band)) return rc;
   // realisations: pairs (2m, 2m + 1) as cg_simulate_pair, a last odd one alone; the posterior
   // means are added in the real domain
   for (int r = 0; r < v->nreal && !rc; r += 2) {

@@ -16,6 +16,8 @@
 // The plans (n, TPS, radices) come from cg_fft_plans.h.
 #pragma once
 
+#include <type_traits>
+
 #include "cg_colour.h"
 #include "cg_dft.h"
 #include "cg_fft_plans.h"
@@ -103,7 +105,8 @@ struct Stages<N, DIR, TPS, ES, NS, P, RS...> {
 // inputs straight from global memory and store the last stage's outputs straight back, which
 // saves two LDS round trips and two barriers per tile).
 //   First<P1>::Regs<BPT1>: v[b][q] = element (t + b TPS) + q N/P1 of the sequence.
-//   sink(e, value) receives element e of the transformed sequence.
+//   sink(e, value) receives element e of the transformed sequence; a sink of four arguments also
+//   the last stage's butterfly b and output q (e = t + b TPS + q N/P of that stage).
 template <int N, int DIR, int TPS, int ES, int NS, int... RS>
 struct StagesIO;
 
@@ -137,7 +140,8 @@ struct StagesIO<N, DIR, TPS, ES, NS, P, RS...> {
         const int d = (j / NS) * NS * P + k;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-          if constexpr (LAST) sink(d + q * NS, v[b][q]);
+          if constexpr (LAST && std::is_invocable_v<Sink &, int, float2, int, int>) sink(d + q * NS, v[b][q], b, q);
+          else if constexpr (LAST) sink(d + q * NS, v[b][q]);
           else buf[(d + q * NS) * ES] = v[b][q];
         }
       }
@@ -165,12 +169,21 @@ struct StagesIO<N, DIR, TPS, ES, NS, P, RS...> {
   }
 };
 
+// The last of a plan's radices.
+template <int R, int... RS>
+constexpr int last_radix()
+{
+  if constexpr (sizeof...(RS) == 0) return R;
+  else return last_radix<RS...>();
+}
+
 template <int N>
 struct Plan;
 #define CG_PLAN(n, tps, ...)                                                                    \
   template <>                                                                                   \
   struct Plan<n> {                                                                              \
     static constexpr int TPS = tps;                                                             \
+    static constexpr int LAST = last_radix<__VA_ARGS__>();                                      \
     template <int DIR, int ES>                                                                  \
     static __device__ __forceinline__ void run(float2 *b, int t, const float2 *w)               \
     {                                                                                           \

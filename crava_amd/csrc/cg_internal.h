@@ -60,6 +60,21 @@ struct XArgs {
   float scale;
 };
 
+// One grid of a band-limited pass (cg_band.h).
+struct BandArgs {
+  const float *real;  // z forward: the real grid read; z inverse: the real grid added
+  float2 *band;       // the band's planes [nb][nyp][rnxp] (x forward: in place when band_out is band)
+  float2 *band_out;   // x passes: where the rows go
+  float *out;         // z inverse: the real grid written
+  const int *kb;      // [nb] the band's frequencies, ascending, 0..nzp/2
+  const int *at;      // [nzp/2 + 1] the band's plane of a frequency, or -1
+  long rows;          // nb nyp
+  unsigned nb, ncols, cnxp;  // ncols = cnxp nyp float pairs per plane
+  int nxp;
+  unsigned block0;
+  float scale;
+};
+
 // Registry of compiled lengths: kind STRIDED (y/z, n = axis length), XE (even nxp, n = nxp/2),
 // XO (odd nxp, n = nxp); `tile` is TI columns (STRIDED) or RW rows (XE/XO) per workgroup.
 enum { FIX_STRIDED = 0, FIX_XE = 1, FIX_XO = 2, FIX_KINDS = 3 };
@@ -73,6 +88,7 @@ typedef int (*ColourZFn)(cg_ctx *, const ColourParams *one, const ColourItem *it
                          const float2 *tw);
 typedef int (*ColourZ2Fn)(cg_ctx *, const ColourParams *one, const ColourItem *items, int nitems, unsigned nblocks,
                           const float2 *tw);
+typedef int (*BandFn)(cg_ctx *, int dir, const BandArgs *items, int nitems, unsigned nblocks, const float2 *tw);
 struct FixedEntry {
   int kind, n;
   int tile[2];  // the two tile variants (equal when the length has only one)
@@ -84,6 +100,8 @@ struct FixedEntry {
   int tune;      // 0: variant 0 is kept (the autotuner's timing on scratch grids misjudges it)
   ColourZ2Fn cz2;  // strided lengths: two realisations per launch (fused colouring)
   int cz2_tile;    // its columns per workgroup
+  BandFn bz, bx;   // strided lengths: band-limited z pass (n = nzp) and x pass (n = nxp)
+  int bz_tile, bx_rows;  // their columns and rows per workgroup
 };
 // Tile variant for a pass geometry: the autotuner's choice (cg_autotune) for this exact
 // geometry, or the context's forced variant, else 0.  `geom` identifies the pass: strided

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "cg_internal.h"
+#include "cg_noise.h"
 
 #include <cstdint>
 
@@ -81,6 +82,16 @@ struct ColourParams;
 // (optional, [3]): posterior means in that layout, added.
 int colour_split(cg_ctx *ctx, const ColourParams &p, int n1, int n2, bool pair,
                  const float2 *const *mean_split = nullptr);
+// The posterior of a band-limited inversion (cg_band.h): mean[] and data[] hold the band's planes,
+// cov[] receive the covariance spectra of every plane, mean[] the update m' - m of the band's
+// wavenumbers (zero where the prior is kept).
+struct PostBandArgs {
+  PostParams p;
+  const int *at;     // [nzp/2 + 1] the band's plane of a frequency, or -1
+  FastDiv by_cnxp;
+  unsigned rnxp;     // pitch of a band row
+};
+int launch_posterior_band(cg_ctx *ctx, const PostBandArgs &b);
 // The allocation-free variant's fixed device buffer (cg_posterior_noalloc): one per device, a
 // file-scope array of kNoAllocBytes; noalloc_scratch_init looks up its address on the current
 // device once (at context creation), noalloc_scratch returns it (null before the lookup or if it

@@ -296,6 +296,158 @@ void launch_nt64(const cg::PostParams &p, unsigned blocks, hipStream_t s, bool s
   }
 }
 
+// ---------------------------------------------------------------- band-limited inversions
+// One wavenumber (cell c = i + cnxp j of plane k) in the band layout (cg_band.h): planes k <= nzp/2
+// read and write W[b][j][i], planes above it the conjugate of W[b][-j][-i], the columns 0 and (even
+// nxp) nxp/2 through their copies past nxp.  A plane that is its own mirror writes both.
+struct BandCell {
+  size_t own, twin;  // W index of the cell; of its conjugate partner (self-mirrored planes)
+  bool conj, self;
+};
+
+__device__ __forceinline__ BandCell band_cell(const cg::PostBandArgs &g, int k, unsigned c, int b)
+{
+  const cg::PostParams &p = g.p;
+  const unsigned j = cg::fast_div(c, g.by_cnxp), i = c - j * (unsigned)p.cnxp;
+  const unsigned jm = j ? (unsigned)p.nyp - j : 0u;
+  const unsigned im = i == 0 ? (unsigned)p.nxp : 2 * i == (unsigned)p.nxp ? (unsigned)p.nxp + 1u : (unsigned)p.nxp - i;
+  const size_t plane = (size_t)b * p.nyp * g.rnxp;
+  const size_t direct = plane + (size_t)j * g.rnxp + i, mirror = plane + (size_t)jm * g.rnxp + im;
+  BandCell x;
+  x.self = k == 0 || 2 * k == p.nzp;
+  x.conj = !x.self && 2 * k > p.nzp;
+  x.own = x.conj ? mirror : direct;
+  x.twin = mirror;
+  return x;
+}
+
+template <typename R>
+__device__ __forceinline__ cpx<R> band_get(const float2 *w, const BandCell &x)
+{
+  const float2 v = gld(w + x.own);
+  return mk<R>(v.x, x.conj ? -v.y : v.y);
+}
+__device__ __forceinline__ void band_put(float2 *w, const BandCell &x, float2 v)
+{
+  gst(w + x.own, make_float2(v.x, x.conj ? -v.y : v.y));
+  if (x.self) gst(w + x.twin, make_float2(v.x, -v.y));
+}
+
+// post32_body (separable prior, host lambda table, no residual) in the band layout.
+template <int NT, bool MIXED>
+__global__ void __launch_bounds__(cg::kThreads) k_posterior_band(cg::PostBandArgs g)
+{
+  const cg::PostParams &p = g.p;
+  const int k = blockIdx.y;
+  const unsigned plane = (unsigned)p.cnxp * (unsigned)p.nyp;
+  const unsigned c = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool active = c < plane;
+  const unsigned cc = active ? c : 0u;
+  const long idx = (long)k * plane + cc;
+  const int b = kat(g.at, 2 * k <= p.nzp ? k : p.nzp - k);  // wavefront-uniform
+  const bool inv = kat(p.invert, k) != 0;
+  bool did_inv = false, did_fail = false, defer = false;
+  if (active) {
+    float P6[6];
+    const float r = prior6<true>(p, idx, cc, k, P6);
+    bool keep = !inv;
+    const BandCell x = band_cell(g, k, cc, b < 0 ? 0 : b);
+    if (inv) {
+      did_inv = true;
+      const float lt = gld(p.lam2d + cc);
+      const float lam = sqrtf(lt * lt);
+      cpx<float> m3[3], d[NT], cov6[6], res[NT];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) m3[a] = band_get<float>(p.mean[a], x);
+#pragma unroll
+      for (int l = 0; l < NT; ++l) d[l] = band_get<float>(p.data[l], x);
+      float cond = 0.f;
+      const int fail = update<NT, float, true, true>(kat(p.tab32, k), r, lam, P6, m3, d, cov6, res, false, cond);
+      if (MIXED && (fail || cond > p.cond_limit)) {
+        defer = true;
+      } else if (fail) {  // posterior = prior (avoinversion.cpp:1040-1042)
+        did_fail = true;
+        keep = true;
+      } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) band_put(p.mean[a], x, make_float2(m3[a].re, m3[a].im));
+#pragma unroll
+        for (int q = 0; q < 6; ++q) gst(p.cov[q] + idx, make_float2(cov6[q].re, cov6[q].im));
+      }
+    }
+    if (keep) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) gst(p.cov[q] + idx, make_float2(P6[q], 0.f));
+      if (b >= 0) {  // an inverted plane's cell, or the mirror of one that is not inverted itself
+#pragma unroll
+        for (int a = 0; a < 3; ++a) band_put(p.mean[a], x, make_float2(0.f, 0.f));
+      }
+    }
+  }
+  if (MIXED) {  // wave-aggregated append to the FP64 list, as post32_body
+    const unsigned long long m = __ballot(defer);
+    if (m) {
+      unsigned long long base = 0;
+      if (__lane_id() == 0) base = atomicAdd(p.list_len, (unsigned long long)__popcll(m));
+      base = __shfl(base, 0);
+      const unsigned lane = __lane_id();
+      const unsigned long long below = lane ? (m & ((~0ull) >> (64 - lane))) : 0ull;
+      if (defer) gst(p.list + (base + __popcll(below)), (unsigned)idx);
+    }
+  }
+  if (p.stats) {
+    wave_count(p.stats, did_inv);
+    wave_count(p.stats + 64, did_fail);
+  }
+}
+
+// post64_cell in the band layout, over the deferred list.
+template <int NT>
+__global__ void __launch_bounds__(cg::kThreads) k_posterior64_band(cg::PostBandArgs g)
+{
+  const cg::PostParams &p = g.p;
+  const unsigned plane = (unsigned)p.cnxp * (unsigned)p.nyp;
+  const unsigned long long n = *p.list_len;
+  for (unsigned long long e = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; e < n;
+       e += (unsigned long long)gridDim.x * blockDim.x) {
+    const unsigned idx = gld(p.list + e);
+    const int k = (int)(idx / plane);
+    const unsigned c = idx - (unsigned)k * plane;
+    const BandCell x = band_cell(g, k, c, kat(g.at, 2 * k <= p.nzp ? k : p.nzp - k));
+    float P6[6];
+    prior6<true>(p, (long)idx, c, k, P6);
+    const double rd = fabs((double)gld(p.rxy + c) * (double)kat(p.rt, k)), lam = fabs((double)gld(p.lam2d + c));
+    double P6d[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) P6d[q] = rd * p.s6d[q];
+    cpx<double> m3[3], d[NT], cov6[6], res[NT];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) m3[a] = band_get<double>(p.mean[a], x);
+#pragma unroll
+    for (int l = 0; l < NT; ++l) d[l] = band_get<double>(p.data[l], x);
+    double cond = 0.0;
+    const int fail = update<NT, double, true, true>(kat(p.tab64, k), rd, lam, P6d, m3, d, cov6, res, false, cond);
+    if (fail && p.stats) atomicAdd(p.stats + 64, 1ull);  // rare: the FP64 factor failed too
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      band_put(p.mean[a], x, fail ? make_float2(0.f, 0.f) : make_float2((float)m3[a].re, (float)m3[a].im));
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      gst(p.cov[q] + idx, fail ? make_float2(P6[q], 0.f) : make_float2((float)cov6[q].re, (float)cov6[q].im));
+  }
+}
+
+template <int NT>
+void launch_band_nt(const cg::PostBandArgs &g, dim3 grid, hipStream_t s, bool mixed)
+{
+  if (mixed) {
+    k_posterior_band<NT, true><<<grid, cg::kThreads, 0, s>>>(g);
+    k_posterior64_band<NT><<<1024, cg::kThreads, 0, s>>>(g);
+  } else {
+    k_posterior_band<NT, false><<<grid, cg::kThreads, 0, s>>>(g);
+  }
+}
+
 // The allocation-free posterior's buffer: device memory of fixed size on every device the library
 // runs on, held until the process ends.  Host code never passes this name to a kernel (in host
 // code it is only a stand-in for the symbol); it uses the address noalloc_scratch_init looked up.
@@ -364,6 +516,27 @@ int zero_words(cg_ctx *ctx, unsigned long long *d, size_t n)
   if (b > 4096) b = 4096;
   k_zero_words<<<(unsigned)b, kThreads, 0, ctx->stream>>>(d, (unsigned long long)n);
   return hip_fail(ctx, hipGetLastError(), "k_zero_words");
+}
+
+int launch_posterior_band(cg_ctx *ctx, const PostBandArgs &b)
+{
+  const long plane = (long)b.p.cnxp * b.p.nyp;
+  const dim3 grid((unsigned)((plane + kThreads - 1) / kThreads), (unsigned)b.p.nzp);
+  const bool mixed = b.p.precision == CG_PREC_MIXED;
+  hipEvent_t ev;
+  launch_begin(ctx, CG_K_POSTERIOR, &ev);
+  switch (b.p.nt) {
+    case 1: launch_band_nt<1>(b, grid, ctx->stream, mixed); break;
+    case 2: launch_band_nt<2>(b, grid, ctx->stream, mixed); break;
+    case 3: launch_band_nt<3>(b, grid, ctx->stream, mixed); break;
+    case 4: launch_band_nt<4>(b, grid, ctx->stream, mixed); break;
+    case 5: launch_band_nt<5>(b, grid, ctx->stream, mixed); break;
+    case 6: launch_band_nt<6>(b, grid, ctx->stream, mixed); break;
+    case 7: launch_band_nt<7>(b, grid, ctx->stream, mixed); break;
+    default: launch_band_nt<8>(b, grid, ctx->stream, mixed); break;
+  }
+  launch_end(ctx, CG_K_POSTERIOR, ev);
+  return hip_fail(ctx, hipGetLastError(), "k_posterior_band");
 }
 
 int launch_posterior(cg_ctx *ctx, const PostParams &p)

@@ -109,8 +109,9 @@ __device__ __forceinline__ void lsolve(const cpx<R> (&L)[NT * (NT + 1) / 2], con
 //   (K Sigma_m)^H M^-1 (K Sigma_m) = Y^H Y,   X^H r = Y^H (L^-1 r)   (X = M^-1 K Sigma_m),
 // which is the reference's M^-1 solve (lib_matrAXeqBMatCpx, forward then backward
 // substitution) rearranged so that only forward substitutions remain.
-// Returns 0 on success (outputs written), 1 on Cholesky failure (outputs untouched).
-template <int NT, typename R, bool SEP, class Tab>
+// Returns 0 on success (outputs written), 1 on Cholesky failure (outputs untouched).  DELTA: m3
+// receives m' - m instead of m'.
+template <int NT, typename R, bool SEP, bool DELTA = false, class Tab>
 __device__ __forceinline__ int update(const Tab &T, R r, R lam, const R (&P6)[6], cpx<R> (&m3)[3],
                                       cpx<R> (&d)[NT], cpx<R> (&cov6)[6], cpx<R> (&res)[NT], bool want_res,
                                       R &cond_lb)
@@ -200,8 +201,8 @@ __device__ __forceinline__ int update(const Tab &T, R r, R lam, const R (&P6)[6]
       xr = fmr(Y[a][l].re, z[l].re, fmr(Y[a][l].im, z[l].im, xr));
       xi = fmr(Y[a][l].re, z[l].im, fmr(-Y[a][l].im, z[l].re, xi));
     }
-    m3[a].re = fmr(s1, xr, m3[a].re);
-    m3[a].im = fmr(s1, xi, m3[a].im);
+    m3[a].re = DELTA ? s1 * xr : fmr(s1, xr, m3[a].re);
+    m3[a].im = DELTA ? s1 * xi : fmr(s1, xi, m3[a].im);
   }
   if (want_res) {
 #pragma unroll

@@ -456,8 +456,10 @@ int cg_batch_destroy(cg_batch *batch);
  * cg_simulate_pair; the posterior means added in the real domain).  Where the grid has a compiled
  * split nzp = 16 N2 for its x length and the call uses the separable prior with host tables
  * (rxy, rt, lam2d) and no residual, the z transform runs in two stages carried by the x passes
- * and the posterior pass (fewer passes over HBM, same results to FP32 rounding); otherwise the
- * drop-in sequence (cg_fft_r2c, cg_posterior, cg_fft_c2r_inplace) runs.  On return post.mean[]
+ * and the posterior pass (fewer passes over HBM, same results to FP32 rounding); large grids of the
+ * same kind of call whose inverted planes are few (about 60 to 75% of all) transform only the
+ * inverted frequencies and add the update to the prior mean (same results to FP32 rounding);
+ * otherwise the drop-in sequence (cg_fft_r2c, cg_posterior, cg_fft_c2r_inplace) runs.  On return post.mean[]
  * hold the real-domain posterior means and post.cov[] the posterior covariance spectra;
  * post.data[] are work grids whose contents are unspecified unless want_residual (then the
  * residual spectra).  post.stats as for cg_posterior. */

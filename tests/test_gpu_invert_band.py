@@ -1,0 +1,103 @@
+"""cg_invert's band-limited passes (large grids whose inverted planes are few): only the inverted
+frequencies go through the x and y passes, the update comes back and is added to the prior mean.
+Against the drop-in sequence on the runtime-plan FFT engine, which computes every wavenumber: odd
+and even lengths on every axis, lengths with and without a two-radix split, the longest tables,
+planes that are their own mirror, inverted planes whose mirror is not, tables without Hermitian
+symmetry (the half-complex inverse keeps the Hermitian part), FP64 re-solves, failures, one and two
+angles (updates sharing a work grid), realisations.
+
+Covariances depend on the tables alone: bit for bit.  Means: both sides are FP32 transforms of the
+same data, each within about 3e-7 of its largest part; the updates are as large as the means here,
+so 5e-6 of the update covers both."""
+import numpy as np
+import pytest
+
+import crava_amd as C
+import problem as P
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "even": dict(shape=(256, 250, 200), nt=3, nreal=2),
+    "odd": dict(shape=(245, 225, 243), nt=5),
+    "odd x, even z, one angle": dict(shape=(375, 189, 180), nt=1, high=25.0),
+    "two angles": dict(shape=(240, 243, 216), nt=2, nreal=1),
+    "long": dict(shape=(1152, 10, 1120), nt=4),
+    "long odd": dict(shape=(735, 25, 675), nt=3),
+    "eight angles": dict(shape=(280, 216, 225), nt=8, precision=C.PREC_REFERENCE),
+    "self-mirrored planes": dict(shape=(252, 240, 210), nt=3, planes=(0, 105, 1, 209, 30, 180)),
+    "one-sided planes": dict(shape=(250, 245, 200), nt=3, planes=(20, 21, 190, 100)),
+    "re-solves": dict(shape=(256, 250, 200), nt=5, sn=1e8),
+    "failures": dict(shape=(240, 250, 210), nt=3, precision=C.PREC_REFERENCE, fail=True),
+}
+
+
+def _problem(nt, shape, high=55.0, planes=None, sn=5.0, fail=False, **_):
+    nxp, nyp, nzp = shape
+    p = P.make_problem(14, 3, int(nzp * 0.8), nxp=16, nyp=4, nzp=nzp, angles_deg=tuple(np.linspace(0.0, 40.0, nt)),
+                       high_cut=high, sn=sn, seed=nzp)
+    rng = np.random.default_rng(nxp)
+    p.update(nx=nxp - 3, ny=max(nyp - 3, 1), nxp=nxp, nyp=nyp)
+    lateral = np.exp(rng.uniform(-3.0, 1.0, (nyp, nxp // 2 + 1))).astype(np.float32)  # no symmetry
+    p["rxy"], p["lam2d"] = lateral, lateral
+    p["mean_real"] = rng.standard_normal((3, nzp, nyp, nxp), dtype=np.float32)
+    p["seis_real"] = rng.standard_normal((nt, nzp, nyp, nxp), dtype=np.float32)
+    if planes is not None:
+        inv = np.zeros(nzp, np.int32)
+        inv[list(planes)] = 1
+        p["invert"] = inv
+    if fail:
+        p.update(sigma0e=-10.0 * np.abs(p["sigma0e"]) - 1.0, prior_var0=p["prior_var0"] * 1e-12)
+    return p
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_band_matches_dropin(ctx, name):
+    kw = CASES[name]
+    nt, nreal, prec = kw["nt"], kw.get("nreal", 0), kw.get("precision", C.PREC_MIXED)
+    print("band", name, kw, flush=True)
+    p = _problem(**kw)
+    mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=5, mean_in=mk(C.PARAMETER, 3),
+              seis_in=mk(C.DATA, nt), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, nt), cov=mk(C.COVARIANCE, 6),
+              out=[mk(C.PARAMETER, 3) for _ in range(nreal)])
+    for g, r in zip(it["mean_in"] + it["seis_in"], list(p["mean_real"]) + list(p["seis_real"])):
+        g.upload_real(r)
+    res = {}
+    for engine in (C.FFT_GENERIC, C.FFT_AUTO):
+        ctx.set_fft_engine(engine)
+        ctx.set_profiling(True)
+        ctx.reset_kernel_time()
+        try:
+            stats = C.invert(ctx, it, precision=prec, stats=True)
+            ctx.sync()
+            passes = ctx.kernel_time(C.K_FFT_Z)[0]
+        finally:
+            ctx.set_profiling(False)
+            ctx.set_fft_engine(C.FFT_AUTO)
+        res[engine] = (np.stack([g.download_real(padded=True) for g in it["mean"]]),
+                       [g.download_complex() for g in it["cov"]],
+                       [np.stack([g.download_real() for g in r]) for r in it["out"]], stats, passes)
+    (m0, c0, o0, s0, _), (m1, c1, o1, s1, z1) = res[C.FFT_GENERIC], res[C.FFT_AUTO]
+    assert s1 == s0
+    if kw.get("sn"):
+        assert s1[2] > s1[0] // 2
+    if kw.get("fail"):
+        assert s1[0] == s1[1] > 0
+    assert all(np.array_equal(a, b) for a, b in zip(c0, c1))
+    nxp = p["nxp"]
+    assert not np.any(m1[..., nxp:])  # the row padding is zero, as the inverse transform leaves it
+    base = p["mean_real"]
+    if kw.get("fail"):
+        assert np.array_equal(m1[..., :nxp], base)  # no update: the prior mean as it was
+        assert rel_l2(m0[..., :nxp], base) < 1e-6
+    else:
+        e = rel_l2(m1[..., :nxp] - base, m0[..., :nxp] - base)
+        print("band %s: mean update %.2e, stats %s, z launches %d" % (name, e, s1, z1), flush=True)
+        # re-solved wavenumbers amplify the rounding of the data (S/N 1e8)
+        assert e < (5e-3 if kw.get("sn") else 5e-6)
+    for a, b in zip(o0, o1):
+        assert rel_l2(b, a) < 5e-6
+    for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"] + [g for r in it["out"] for g in r]:
+        g.close()
