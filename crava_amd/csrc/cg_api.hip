@@ -1512,11 +1512,11 @@ int cg_simulate_pair(cg_ctx *ctx, const cg_sim_args *a, cg_grid *next_out[3])
 }
 
 // ---------------------------------------------------------------------------- passes over several grids
-// The FFT passes of several grids of one geometry in shared launches (descriptor lists), the same
-// kernels and tile variants as grid by grid, so the same bits.  A small grid's pass does not fill
+// The FFT passes of several grids of one geometry in shared launches (descriptor lists), with the
+// kernels and tile variants of a batch, so that an inversion has the same bits alone and batched.  A small grid's pass does not fill
 // the device (64 x 64 x 128 padded to 84 x 84 x 180: 945 workgroups of one wavefront, 9 us for
 // 2 us of traffic), and a request is dozens of them: with 3 angles and a realisation 39 launches
-// and 313 us grid by grid, 13 launches and 179 us in lists.
+// and 313 us grid by grid, 13 launches and 166 us in lists.
 }  // extern "C"
 
 namespace {

@@ -225,8 +225,8 @@ constexpr int strided_tile()
 
 // x pass, variant 0: the most rows (up to 128) whose LDS (N twiddles + (N + 1)(RW + 1) slots)
 // fits kLds with at most 512 threads; variant 1: half as many rows (more workgroups per CU).
-// Even nxp, where x_rows_dma allows it: variant 0 is the double-buffered kernel, variant 1 the
-// single-buffered one with x_rows<N, 0>() rows.
+// Even nxp: variant 0 is the wavefront kernel (k_rowe) where the half-length has a two-radix split,
+// else the double-buffered one where x_rows_dma allows it; variant 1 the single-buffered one.
 template <int N, int V>
 constexpr int x_rows()
 {
@@ -237,11 +237,20 @@ constexpr int x_rows()
 }
 template <int N>
 constexpr int x_rows_dma();
-// Rows per tile of variant V of the even-nxp x pass.
+template <int N>
+struct Row;
+template <int N, int V>
+constexpr int xe_rows_plan()
+{
+  return x_rows_dma<N>() > 0 ? (V == 0 ? x_rows_dma<N>() : x_rows<N, 0>()) : x_rows<N, V>();
+}
+// Rows per tile of variant V of the even-nxp x pass (variant 2: the drop-in forward pass).
 template <int N, int V>
 constexpr int xe_rows()
 {
-  return x_rows_dma<N>() > 0 ? (V == 0 ? x_rows_dma<N>() : x_rows<N, 0>()) : x_rows<N, V>();
+  if (V == 0 && Row<N>::OK) return Row<N>::SEQS;
+  if (V == 2) return xe_rows_plan<N, 0>();
+  return xe_rows_plan<N, V>();
 }
 
 __device__ __forceinline__ void load_tw(float2 *tw, const float2 *g, int n, int tid, int nthr)
@@ -477,8 +486,187 @@ k_fftx_c2r(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const
   }
 }
 
+// ---------------------------------------------------------------- x pass, rows in a wavefront
+// The even-nxp x pass of the half-lengths that split into two radices P1 P2 <= 32 (row_split).  A row
+// belongs to T = P2 lanes of one wavefront, R = 64 / T rows to a wavefront: the first radix stage
+// takes its inputs straight from global memory (a row's lanes on consecutive elements), one exchange
+// through the wavefront's own LDS (element q of lane t at q PITCH + t, read back at t PITCH + q:
+// PITCH is odd, so neither side conflicts) feeds the second stage, whose outputs go straight back.
+// The pairs (k, N - k) of the real transform sit in lanes t and P - t with mirrored registers, so the
+// R2C / C2R pass is a cross-lane read.  No workgroup barrier but the one for the twiddles:
+// wavefronts drift apart, and their loads, arithmetic and stores overlap.  The double-buffered
+// kernel below holds two row sets in LDS (5 wavefronts per CU at any length, half a wavefront per
+// workgroup at the shortest); this one holds none while loading (16 per CU).  Measured, microseconds
+// per launch, double-buffered / this (forward, inverse, inverse + add; the last column in TB/s):
+//   nxp 576, 576 x 320 rows    171 / 165   183 / 185   263 / 259   4.9-5.2
+//   nxp 280, 270 x 243 rows   38.3 / 37.4  39.9 / 35.2 52.4 / 48.7 4.0-4.6
+//   nxp 224, 280 x 200 rows   30.4 / 26.6  33.5 / 25.2 42.0 / 36.7 3.8-4.1
+//   nxp 84,  84 x 180 rows     7.4 / 4.3    8.9 / 4.7  10.1 / 5.1  2.2-3.1
+// Memory bounds it at the long lengths (128-byte stores at rows' odd pitch), latency at the short.
+constexpr int row_split(int n)  // P1 (<= P2 = n / P1): the factors closest to sqrt(n); 0: none
+{
+  int best = 0;
+  for (int p = 1; p <= 32; ++p)
+    if (n % p == 0 && p * p <= n && n / p <= 32) best = p;
+  return best;
+}
+
+template <int N>
+struct Row {
+  static constexpr int P1 = row_split(N);
+  static constexpr bool OK = P1 > 0;
+  static constexpr int P2 = OK ? N / (OK ? P1 : 1) : 1;
+  static constexpr int T = P2;           // lanes per sequence
+  static constexpr int R = 64 / T;       // sequences per wavefront
+  static constexpr int WAVES = 4;        // wavefronts per workgroup
+  static constexpr int SEQS = WAVES * R;
+  static constexpr int PITCH = P2 | 1;
+  static constexpr int LDS = R * P1 * PITCH;  // float2 per wavefront
+};
+
+// Keeps the compiler from moving LDS accesses across the exchange.  The hardware needs nothing:
+// a wavefront's LDS operations complete in order.
+__device__ __forceinline__ void wave_lds_order()
+{
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float2 lane_read(int lane4, float2 v)  // lane4: source lane times 4
+{
+  return make_float2(__int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(v.x))),
+                     __int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(v.y))));
+}
+
+// v[q] = element t + q P2 of the sequence (lanes t < P2); returns u[q] = element t + q P1 of its
+// transform (lanes t < P1).  tw: w^m of length N M in LDS.
+template <int N, int DIR, int M>
+__device__ __forceinline__ void row_fft(float2 (&v)[Row<N>::P1], float2 (&u)[Row<N>::P2], float2 *buf, int t,
+                                        bool on, const float2 *tw)
+{
+  using P = Row<N>;
+  if (on) {
+    dft<DIR, P::P1>(v);
+#pragma unroll
+    for (int q = 0; q < P::P1; ++q) buf[q * P::PITCH + t] = v[q];
+  }
+  wave_lds_order();
+  if (on && t < P::P1) {
+#pragma unroll
+    for (int q = 0; q < P::P2; ++q) u[q] = buf[t * P::PITCH + q];
+    if (P::P1 > 1) {
+#pragma unroll
+      for (int q = 1; q < P::P2; ++q) {
+        float2 w = tw[q * t * M];
+        if (DIR > 0) w.y = -w.y;
+        u[q] = cmul(u[q], w);
+      }
+    }
+    dft<DIR, P::P2>(u);
+  }
+}
+
+// Z[N - k] for k = t + q P (a sequence of P Q values held as register q of lane t < P): register
+// Q - 1 - q of lane P - t, and for t = 0 register Q - q of the lane itself (Z[0] for q = 0).
+template <int P, int Q>
+__device__ __forceinline__ float2 row_mirror(const float2 (&z)[Q], int q, int t, int from4)
+{
+  const float2 a = z[(Q - q) % Q], b = z[Q - 1 - q];
+  return lane_read(from4, make_float2(t == 0 ? a.x : b.x, t == 0 ? a.y : b.y));
+}
+
+template <int N, bool FWD, bool ADD>
+__global__ void __launch_bounds__(64 * Row<N>::WAVES)
+k_rowe(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const float2 *__restrict__ tw_row)
+{
+  using P = Row<N>;
+  constexpr int P1 = P::P1, P2 = P::P2, CN = N + 1;
+  __shared__ float2 tw[2 * N];
+  __shared__ float2 lds[P::WAVES][P::LDS];
+  cg::XArgs a;
+  const unsigned blk = resolve(one, items, nitems, a);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = lane / P::T, t = lane - r * P::T;
+  const long row = (long)blk * P::SEQS + (tid >> 6) * P::R + r;
+  const bool on = r < P::R && row < a.rows;
+  float2 *out = reinterpret_cast<float2 *>(a.dst) + (on ? row * CN : 0);
+  const float2 *in = FWD ? reinterpret_cast<const float2 *>(a.src) + (on ? row * CN : 0) : out;
+  float2 v[P1], u[P2], xn = make_float2(0.f, 0.f);
+  if (on) {
+#pragma unroll
+    for (int q = 0; q < P1; ++q) v[q] = cg::gld(in + t + q * P2);
+    if (!FWD && t == 0) xn = cg::gld(in + N);
+  }
+  load_tw(tw, tw_row, 2 * N, tid, 64 * P::WAVES);
+  lds_sync();
+  float2 *buf = lds[tid >> 6] + (r < P::R ? r : 0) * P1 * P::PITCH;
+  if (FWD) {
+    row_fft<N, -1, 2>(v, u, buf, t, on, tw);
+    if (on && t < P1) {
+      const int from4 = 4 * (r * P::T + (t == 0 ? 0 : P1 - t));
+      const float scale = a.scale;
+#pragma unroll
+      for (int q = 0; q < P2; ++q) {  // as k_fftx_r2c: X[k] from (Z[k], conj Z[N-k])
+        const int k = t + q * P1;
+        const float2 za = u[q], zb = row_mirror<P1, P2>(u, q, t, from4);
+        const float2 ea = cscale(cadd(za, cconj(zb)), 0.5f), da = csub(za, cconj(zb));
+        const float2 xa = cadd(ea, cmul(tw[k], make_float2(0.5f * da.y, -0.5f * da.x)));
+        cg::gst(out + k, cscale(xa, scale));
+        if (q == 0 && t == 0) cg::gst(out + N, make_float2(scale * (za.x - za.y), 0.f));
+      }
+    }
+    return;
+  }
+  if (on) {  // as k_fftx_c2r; registers s and P1 - 1 - s of lanes t and P2 - t together
+    const int from4 = 4 * (r * P::T + (t == 0 ? 0 : P2 - t));
+    auto pre = [&](float2 xa, float2 xb, int k) {
+      if (k == 0) {
+        xa.y = 0.f;
+        xb.y = 0.f;
+      }
+      const float2 ea = cadd(xa, cconj(xb)), oa = cmul(csub(xa, cconj(xb)), cconj(tw[k]));
+      return make_float2(ea.x - oa.y, ea.y + oa.x);
+    };
+    float2 above = xn;  // X[P1 - s] of lane 0 before it was replaced (X[N] for s = 0)
+#pragma unroll
+    for (int s = 0; s < (P1 + 1) / 2; ++s) {
+      const int h = P1 - 1 - s;
+      const float2 lo = v[s], hi = v[h];
+      const float2 plo = lane_read(from4, make_float2(t == 0 ? above.x : hi.x, t == 0 ? above.y : hi.y));
+      if (h != s) {
+        const float2 nx = v[s + 1];
+        const float2 phi = lane_read(from4, make_float2(t == 0 ? nx.x : lo.x, t == 0 ? nx.y : lo.y));
+        v[h] = pre(hi, phi, t + h * P2);
+      }
+      v[s] = pre(lo, plo, t + s * P2);
+      above = hi;
+    }
+  }
+  row_fft<N, +1, 2>(v, u, buf, t, on, tw);
+  if (on && t < P1) {
+    const float2 *ad = ADD ? reinterpret_cast<const float2 *>(a.add) + row * CN : nullptr;
+    float2 va[ADD ? P2 : 1];
+    if (ADD) {
+#pragma unroll
+      for (int q = 0; q < P2; ++q) va[ADD ? q : 0] = cg::gld(ad + t + q * P1);
+    }
+#pragma unroll
+    for (int q = 0; q < P2; ++q) {
+      float2 x = cscale(u[q], a.scale);
+      if (ADD) {
+        x.x += va[ADD ? q : 0].x;
+        x.y += va[ADD ? q : 0].y;
+      }
+      cg::gst(out + t + q * P1, x);
+    }
+    if (t == 0) cg::gst(out + N, make_float2(0.f, 0.f));
+  }
+}
+
 // ---------------------------------------------------------------- x pass, double-buffered
-// Even nxp, the second tile variant.  Persistent workgroups (a multiple of 8, as many as the CUs
+// Even nxp: the half-lengths without a two-radix split, and the forward pass of the drop-in
+// transforms at every length (variant 2, see fixed_x).  Persistent workgroups (a multiple of 8, as many as the CUs
 // hold): workgroup b serves XCD b % 8, which walks its eighth of the tiles (a contiguous band)
 // in steps of gridDim.x / 8.  Two LDS tile buffers hold RW rows each in the grid's own layout
 // (row r at r CN, CN = N + 1 odd for even N, so consecutive rows fall on distinct bank pairs):
@@ -1197,21 +1385,31 @@ template <int N, int V>
 int xe_launch(cg_ctx *ctx, int forward, int add, const cg::XArgs *one, const cg::XArgs *items, int nitems,
               unsigned nblocks, const float2 *tw, const float2 *twr)
 {
-  if constexpr (V == 0 && x_rows_dma<N>() > 0) {
+  if constexpr (V == 0 && Row<N>::OK) {
+    constexpr int NT = 64 * Row<N>::WAVES;
+    const cg::XArgs o = one ? *one : cg::XArgs{};
+    if (forward) k_rowe<N, true, false><<<nblocks, NT, 0, ctx->stream>>>(o, items, nitems, twr);
+    else if (add) k_rowe<N, false, true><<<nblocks, NT, 0, ctx->stream>>>(o, items, nitems, twr);
+    else k_rowe<N, false, false><<<nblocks, NT, 0, ctx->stream>>>(o, items, nitems, twr);
+    return cg::hip_fail(ctx, hipGetLastError(), "k_rowe");
+  } else if constexpr (V == 2 && x_rows_dma<N>() > 0) {
+    return xdma_launch<N, true, false>(ctx, one, items, nitems, nblocks, tw, twr);  // forward only
+  } else if constexpr (V == 0 && x_rows_dma<N>() > 0) {
     if (forward) return xdma_launch<N, true, false>(ctx, one, items, nitems, nblocks, tw, twr);
     if (add) return xdma_launch<N, false, true>(ctx, one, items, nitems, nblocks, tw, twr);
     return xdma_launch<N, false, false>(ctx, one, items, nitems, nblocks, tw, twr);
+  } else {
+    constexpr int RW = xe_rows<N, V>();
+    const size_t lds = sizeof(float2) * (N + (size_t)(N + 1) * (RW + 1));
+    const cg::XArgs o = one ? *one : cg::XArgs{};
+    if (forward)
+      k_fftx_r2c<N, RW><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
+    else if (add)
+      k_fftx_c2r<N, RW, true><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
+    else
+      k_fftx_c2r<N, RW, false><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
+    return cg::hip_fail(ctx, hipGetLastError(), "k_fftx");
   }
-  constexpr int RW = xe_rows<N, V>();
-  const size_t lds = sizeof(float2) * (N + (size_t)(N + 1) * (RW + 1));
-  const cg::XArgs o = one ? *one : cg::XArgs{};
-  if (forward)
-    k_fftx_r2c<N, RW><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
-  else if (add)
-    k_fftx_c2r<N, RW, true><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
-  else
-    k_fftx_c2r<N, RW, false><<<nblocks, RW * Plan<N>::TPS, lds, ctx->stream>>>(o, items, nitems, tw, twr);
-  return cg::hip_fail(ctx, hipGetLastError(), "k_fftx");
 }
 
 template <int N, int V>

@@ -91,9 +91,9 @@ typedef int (*ColourZ2Fn)(cg_ctx *, const ColourParams *one, const ColourItem *i
 typedef int (*BandFn)(cg_ctx *, int dir, const BandArgs *items, int nitems, unsigned nblocks, const float2 *tw);
 struct FixedEntry {
   int kind, n;
-  int tile[2];  // the two tile variants (equal when the length has only one)
+  int tile[3];  // the two tile variants (equal when the length has only one); 2: see x
   StridedFn s[2];
-  XFn x[2];
+  XFn x[3];     // [2]: even nxp, the forward pass of the drop-in transforms
   ColourZFn cz;  // strided lengths: colouring fused with the inverse z pass
   int cz_waves;  // wavefronts of the fused kernel resident per CU
   int cz_tile;   // its columns per workgroup

@@ -1,13 +1,15 @@
-"""cg_invert on small grids runs each FFT pass of its grids in shared launches.  The kernels and
-tile variants are those of the grid-by-grid calls, so the results equal the drop-in calls' bit for
-bit: odd and even lengths, single rows and planes, more grids than one launch holds, an odd and an
-even number of realisations, and the means' work grids being the inputs themselves (which the
-shared launches do not take)."""
+"""cg_invert on small grids runs each FFT pass of its grids in shared launches: odd and even lengths,
+single rows and planes, more grids than one launch holds, an odd and an even number of realisations,
+and the means' work grids being the inputs themselves (which the shared launches do not take).
+Against the drop-in calls: bit for bit where they run the same kernels (odd row lengths, and the
+covariances, which depend on the tables alone); even row lengths take another forward x pass, whose
+FP32 rounding (3e-7 of the largest part on either side) the results then carry."""
 import numpy as np
 import pytest
 
 import crava_amd as C
 import problem as P
+from conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -62,7 +64,10 @@ def test_shared_launches_equal_dropin_calls(ctx, case, in_place):
     got = [g.download_real() for g in item["mean"]] + [g.download_complex() for g in cov] + \
           [g.download_real() for r in outs for g in r]
     assert stats == want_stats
-    for w, g in zip(want, got):
-        assert np.array_equal(w, g)
+    for k, (w, g) in enumerate(zip(want, got)):
+        if shape[0] % 2 or in_place or 3 <= k < 9:
+            assert np.array_equal(w, g)
+        else:
+            assert rel_l2(g, w) < 2e-6
     for g in mean_in + seis_in + mean + data + cov + [g for r in outs for g in r]:
         g.close()
