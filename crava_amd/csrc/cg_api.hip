@@ -1668,13 +1668,11 @@ static int invert_band(cg_ctx *ctx, const cg_inversion *v)
   const cg::FixedEntry *ex = cg::fixed_find(cg::FIX_STRIDED, nxp), *ez = cg::fixed_find(cg::FIX_STRIDED, nzp);
   const cg::FixedEntry *ey = nyp > 1 ? cg::fixed_find(cg::FIX_STRIDED, nyp) : nullptr;
   if (!ex || !ez || (nyp > 1 && !ey)) return 1;
-  std::vector<int> kb, at(nzp / 2 + 1, -1);
+  std::vector<int> at(nzp / 2 + 1, -1);
+  size_t nb = 0;  // the band's frequencies
   for (int k = 0; k <= nzp / 2; ++k)
-    if (a.invert[k] || a.invert[k ? nzp - k : 0]) {
-      at[k] = (int)kb.size();
-      kb.push_back(k);
-    }
-  const size_t nb = kb.size(), plane = (size_t)cnxp * nyp, cells = nb * plane * 2;
+    if (a.invert[k] || a.invert[k ? nzp - k : 0]) at[k] = (int)nb++;
+  const size_t plane = (size_t)cnxp * nyp, cells = nb * plane * 2;
   // where the band is worth it, and three updates fit the seismic work grids
   int n1, n2;
   const double most = cg::split_z_supported(nxp, nzp, &n1, &n2) ? kBandMostSplit : kBandMost;
@@ -1721,7 +1719,6 @@ static int invert_band(cg_ctx *ctx, const cg_inversion *v)
     cg::BandArgs b;
     std::memset(&b, 0, sizeof(b));
     b.rows = (long)(nb * nyp);
-    b.nb = (unsigned)nb;
     b.ncols = (unsigned)plane;
     b.cnxp = (unsigned)cnxp;
     b.nxp = nxp;
@@ -1738,28 +1735,25 @@ static int invert_band(cg_ctx *ctx, const cg_inversion *v)
     b.scale = in[g]->cubetype == CG_CT_COVARIANCE ? (fwd ? 1.0f : float(1.0 / (double)N)) : (fwd ? s_fwd : s_inv);
     (fwd ? zf : zi).push_back(b);
   }
-  // the frequency tables and descriptors are staged with the posterior's tables; the descriptors get
-  // the tables' addresses once the layout is known
-  std::vector<std::pair<const void *, size_t>> extra = {{kb.data(), sizeof(int) * nb}, {at.data(), sizeof(int) * at.size()}};
+  // the frequency table and the descriptors are staged with the posterior's tables; the descriptors
+  // get the table's address once the layout is known
+  std::vector<std::pair<const void *, size_t>> extra = {{at.data(), sizeof(int) * at.size()}};
   for (const auto *l : {&zf, &xf, &xi, &zi}) extra.push_back({l->data(), sizeof(cg::BandArgs) * l->size()});
   for (const auto *l : {&yf, &yi}) extra.push_back({l->data(), sizeof(cg::StridedArgs) * l->size()});
   std::vector<void *> dp;
   cg::PostBandArgs pb;
   int rc = post_stage(ctx, &a, extra, dp, pb.p, [&](const std::vector<void *> &d, size_t first) {
     for (auto *l : {&zf, &xf, &xi, &zi})
-      for (auto &b : *l) {
-        b.kb = static_cast<const int *>(d[first]);
-        b.at = static_cast<const int *>(d[first + 1]);
-      }
+      for (auto &b : *l) b.at = static_cast<const int *>(d[first]);
   });
   if (rc) return rc;
   const size_t e0 = dp.size() - extra.size();
-  pb.at = static_cast<const int *>(dp[e0 + 1]);
+  pb.at = static_cast<const int *>(dp[e0]);
   pb.by_cnxp = cg::make_fastdiv((uint32_t)cnxp);
   pb.rnxp = 2u * (unsigned)cnxp;
-  const cg::BandArgs *dz = static_cast<const cg::BandArgs *>(dp[e0 + 2]), *dx = static_cast<const cg::BandArgs *>(dp[e0 + 3]),
-                     *dxi = static_cast<const cg::BandArgs *>(dp[e0 + 4]), *dzi = static_cast<const cg::BandArgs *>(dp[e0 + 5]);
-  const cg::StridedArgs *dy = static_cast<const cg::StridedArgs *>(dp[e0 + 6]), *dyi = static_cast<const cg::StridedArgs *>(dp[e0 + 7]);
+  const cg::BandArgs *dz = static_cast<const cg::BandArgs *>(dp[e0 + 1]), *dx = static_cast<const cg::BandArgs *>(dp[e0 + 2]),
+                     *dxi = static_cast<const cg::BandArgs *>(dp[e0 + 3]), *dzi = static_cast<const cg::BandArgs *>(dp[e0 + 4]);
+  const cg::StridedArgs *dy = static_cast<const cg::StridedArgs *>(dp[e0 + 5]), *dyi = static_cast<const cg::StridedArgs *>(dp[e0 + 6]);
   const float2 *twx = cg::twiddle_table(ctx, nxp), *twz = cg::twiddle_table(ctx, nzp);
   if (!twx || !twz) return CG_ENOMEM;
   auto timed = [&](int kclass, auto f) {

@@ -22,11 +22,44 @@
 
 namespace cgfix {
 
-// Columns (pairs of neighbouring x) per z tile: as the strided passes.
+constexpr int band_split(int n)  // P1 (<= P2 = n / P1): the factors closest to sqrt(n); 0: none
+{
+  int best = 0;
+  for (int p = 1; p <= 32; ++p)
+    if (n % p == 0 && p * p <= n && n / p <= 32) best = p;
+  return best;
+}
+
+// Stages of a z tile.  A length of two radices P1 <= P2 <= 2 P1 runs on TPS = P2 threads per column,
+// the radix P1 on the side that touches memory (forward first, inverse last), so that every thread
+// takes part in the loads or stores with P1 values each; other lengths take their plan.  The plans
+// of the y and z passes hold 20 to 32 values a thread, which leaves few wavefronts per CU once the
+// prior mean's pairs wait in registers too.  Microseconds per grid, plan / this, nzp 384 at 1152 x
+// 576: forward 305 / 292, inverse 1014 / 516 (4.8 TB/s); nzp 360 at 405 x 375: 66.6 / 63.9, 128 / 130;
+// unbalanced radices lose (nzp 243 = 9 x 27 at 280 x 270: 26.6 / 30.9, 44.6 / 47.0).
+template <int N, int DIR, int ES, bool TWO = (band_split(N) > 1 && N <= 2 * band_split(N) * band_split(N))>
+struct BandZ {
+  static constexpr int TPS = Plan<N>::TPS, LAST = Plan<N>::LAST;
+  using IO = typename Plan<N>::template IO<DIR, ES>;
+};
+template <int N, int DIR, int ES>
+struct BandZ<N, DIR, ES, true> {
+  static constexpr int P1 = band_split(N), P2 = N / P1, TPS = P2, LAST = DIR < 0 ? P2 : P1;
+  using IO = StagesIO<N, DIR, TPS, ES, 1, DIR < 0 ? P1 : P2, DIR < 0 ? P2 : P1>;
+};
+
+// Columns (pairs of neighbouring x) per z tile: as the strided passes, with the table of the band's
+// planes in the LDS too.
 template <int N>
 constexpr int band_tile()
 {
-  return strided_tile0<N>();
+  constexpr int ti = strided_tile0<N>();
+  return ti > 8 && sizeof(float2) * N * (ti + 1) + sizeof(short) * (N / 2 + 1) > kLds ? ti / 2 : ti;
+}
+template <int N>
+constexpr int band_threads()
+{
+  return band_tile<N>() * BandZ<N, -1, band_tile<N>()>::TPS;  // the same both ways
 }
 
 // Item of a list (items[i] owns blocks [block0_i, block0_{i+1})).
@@ -39,16 +72,17 @@ __device__ __forceinline__ unsigned band_item(const cg::BandArgs *items, int nit
 
 // z forward.  A column of the grid's float pairs is z = a + i b of two neighbouring traces; after
 // the complex transform A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = -i (Z[k] - conj Z[N-k]) / 2.  The
-// strided pass's tile and stages; the last stage's outputs stay in LDS and the band's frequencies
-// leave as 16-byte pairs (TI of them: 256-byte segments).
+// strided pass's tile; the last stage's outputs stay in LDS and the band's frequencies leave as
+// 16-byte pairs (TI of them: 256-byte segments).  4.4 TB/s at 576 x 576 x 320.
 template <int N>
-__global__ void __launch_bounds__(band_tile<N>() * Plan<N>::TPS)
+__global__ void __launch_bounds__(band_threads<N>())
 k_bandz_fwd(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__restrict__ twg)
 {
-  constexpr int TI = band_tile<N>(), TPS = Plan<N>::TPS, NT = TI * TPS;
-  using IO = typename Plan<N>::template IO<-1, TI>;
+  constexpr int TI = band_tile<N>(), TPS = BandZ<N, -1, TI>::TPS, NT = TI * TPS;
+  using IO = typename BandZ<N, -1, TI>::IO;
   extern __shared__ float2 smem[];
   float2 *tw = smem, *buf = smem + N;
+  __shared__ short at[N / 2 + 1];  // the band's plane of a frequency, or -1
   cg::BandArgs a;
   const unsigned blk = band_item(items, nitems, a);
   const int tid = threadIdx.x, c = tid % TI, t = tid / TI;
@@ -57,6 +91,7 @@ k_bandz_fwd(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
   const bool first = live && 2 * (int)xp < a.nxp, second = live && 2 * (int)xp + 1 < a.nxp;
   const float2 *col = reinterpret_cast<const float2 *>(a.real) + (live ? q : 0);
   load_tw(tw, twg, N, tid, NT);
+  for (int k = tid; k <= N / 2; k += NT) at[k] = (short)cg::gld(a.at + k);
   float2 v[IO::BPT][IO::P_];
 #pragma unroll
   for (int b = 0; b < IO::BPT; ++b) {
@@ -74,28 +109,35 @@ k_bandz_fwd(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
   lds_sync();
   const float s = 0.5f * a.scale;
   typedef float fvec4 __attribute__((ext_vector_type(4)));
-  for (unsigned b = t; b < a.nb; b += TPS) {
-    const int k = cg::gld(a.kb + b);
-    const float2 z = cscale(mine[k * TI], s), m = cscale(mine[(k ? N - k : 0) * TI], s);
-    if (live)
-      *(__attribute__((address_space(1))) fvec4 *)(a.band + 2 * ((size_t)b * a.ncols + q)) =
-          fvec4{z.x + m.x, z.y - m.y, z.y + m.y, m.x - z.x};
+#pragma unroll
+  for (int i = 0; i < (N / 2 + TPS) / TPS; ++i) {  // every frequency 0..N/2, the band's stored
+    const int k = t + i * TPS;
+    const int p = k <= N / 2 ? at[k] : -1;
+    if (p >= 0) {
+      const float2 z = cscale(mine[k * TI], s), m = cscale(mine[(k ? N - k : 0) * TI], s);
+      if (live)
+        *(__attribute__((address_space(1))) fvec4 *)(a.band + 2 * ((size_t)p * a.ncols + q)) =
+            fvec4{z.x + m.x, z.y - m.y, z.y + m.y, m.x - z.x};
+    }
   }
 }
 
 // z inverse: the band's frequencies of two neighbouring columns make Z[k] = A + i B and
 // Z[N-k] = conj A + i conj B (the imaginary parts of a self-conjugate frequency dropped), the rest is
-// zero; the transform's pairs are the two real traces, scaled and added to the prior mean.
+// zero; the transform's pairs are the two real traces, scaled and added to the prior mean.  Every
+// frequency is loaded once and placed in LDS at k and N - k (loading each input of the first stage
+// from memory read the band twice and held 8 of them a thread: 289 -> 221 us per grid at 576 x 576 x
+// 320, 4.6 TB/s).
 template <int N>
-__global__ void __launch_bounds__(band_tile<N>() * Plan<N>::TPS)
+__global__ void __launch_bounds__(band_threads<N>())
 k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__restrict__ twg)
 {
-  constexpr int TI = band_tile<N>(), TPS = Plan<N>::TPS, NT = TI * TPS;
-  using IO = typename Plan<N>::template IO<+1, TI>;
-  constexpr int LP = Plan<N>::LAST, LNB = N / LP, LB = (LNB + TPS - 1) / TPS;  // the last stage's outputs
+  constexpr int TI = band_tile<N>(), TPS = BandZ<N, +1, TI>::TPS, NT = TI * TPS;
+  using IO = typename BandZ<N, +1, TI>::IO;
+  constexpr int LP = BandZ<N, +1, TI>::LAST, LNB = N / LP, LB = (LNB + TPS - 1) / TPS;  // the last stage's outputs
   extern __shared__ float2 smem[];
   float2 *tw = smem, *buf = smem + N;
-  __shared__ int at[N / 2 + 1];  // the band's plane of a frequency, or -1
+  __shared__ short at[N / 2 + 1];  // the band's plane of a frequency, or -1
   cg::BandArgs a;
   const unsigned blk = band_item(items, nitems, a);
   const int tid = threadIdx.x, c = tid % TI, t = tid / TI;
@@ -103,27 +145,18 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
   const bool live = q < a.ncols;
   const bool first = live && 2 * (int)xp < a.nxp, second = live && 2 * (int)xp + 1 < a.nxp;
   load_tw(tw, twg, N, tid, NT);
-  for (int k = tid; k <= N / 2; k += NT) at[k] = cg::gld(a.at + k);
+  for (int k = tid; k <= N / 2; k += NT) at[k] = (short)cg::gld(a.at + k);
   lds_sync();
   typedef float fvec4 __attribute__((ext_vector_type(4)));
   const float2 *src = a.band + 2 * (size_t)(live ? q : 0);
-  float2 v[IO::BPT][IO::P_];
+  // every frequency 0..N/2 once (zero outside the band), all loads in flight
+  constexpr int KPT = (N / 2 + TPS) / TPS;
+  fvec4 f[KPT];
 #pragma unroll
-  for (int b = 0; b < IO::BPT; ++b) {
-    const int j = t + b * TPS;
-#pragma unroll
-    for (int r = 0; r < IO::P_; ++r) {
-      const int k = j + r * IO::NB, kk = 2 * k <= N ? k : N - k;
-      const int p = first && (IO::EVEN || j < IO::NB) ? at[kk] : -1;
-      float2 x = make_float2(0.f, 0.f);
-      if (p >= 0) {
-        const fvec4 f = *(const __attribute__((address_space(1))) fvec4 *)(src + 2 * (size_t)p * a.ncols);
-        if (k == 0 || 2 * k == N) x = make_float2(f.x, f.z);
-        else if (k == kk) x = make_float2(f.x - f.w, f.y + f.z);
-        else x = make_float2(f.x + f.w, f.z - f.y);
-      }
-      v[b][r] = x;
-    }
+  for (int i = 0; i < KPT; ++i) {
+    const int k = t + i * TPS;
+    const int p = first && k <= N / 2 ? at[k] : -1;
+    f[i] = p >= 0 ? *(const __attribute__((address_space(1))) fvec4 *)(src + 2 * (size_t)p * a.ncols) : fvec4{0.f, 0.f, 0.f, 0.f};
   }
   // the prior mean's pairs of this thread's outputs (element j + r LNB of the column), in flight
   // during the transform
@@ -136,6 +169,16 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
     for (int r = 0; r < LP; ++r)
       m[b][r] = (first && (LNB % TPS == 0 || j < LNB)) ? cg::gld(add + (long)(j + r * LNB) * a.ncols) : make_float2(0.f, 0.f);
   }
+  float2 *mine = buf + c;
+#pragma unroll
+  for (int i = 0; i < KPT; ++i) {
+    const int k = t + i * TPS;
+    if (k > N / 2) continue;
+    const bool self = k == 0 || 2 * k == N;
+    mine[k * TI] = self ? make_float2(f[i].x, f[i].z) : make_float2(f[i].x - f[i].w, f[i].y + f[i].z);
+    if (!self) mine[(N - k) * TI] = make_float2(f[i].x + f[i].w, f[i].z - f[i].y);
+  }
+  lds_sync();
   const float scale = a.scale;
   float2 *out = reinterpret_cast<float2 *>(a.out) + (live ? q : 0);
   auto sink = [&](int e, float2 x, int b, int r) {
@@ -145,7 +188,7 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
     if (!second) o.y = 0.f;
     if (live) cg::gst(out + (long)e * a.ncols, o);
   };
-  IO::step(v, buf + c, t, tw, sink);
+  IO::from_lds(mine, t, tw, sink);
 }
 
 // x pass of the band's rows (complex, whole length N = nxp; pitch rnxp).  Lengths that split into
@@ -154,14 +197,6 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
 // q PITCH + t, read back at t PITCH + q, PITCH odd: no bank conflicts), the second stage's outputs
 // go straight back, and no barrier but the one for the twiddles.  The others take the length's
 // plan with a row on TPS threads.
-constexpr int band_split(int n)  // P1 (<= P2 = n / P1): the factors closest to sqrt(n); 0: none
-{
-  int best = 0;
-  for (int p = 1; p <= 32; ++p)
-    if (n % p == 0 && p * p <= n && n / p <= 32) best = p;
-  return best;
-}
-
 template <int N>
 struct BandRow {
   static constexpr int P1 = band_split(N);
@@ -283,8 +318,9 @@ int bandz_launch(cg_ctx *ctx, int dir, const cg::BandArgs *items, int nitems, un
 {
   constexpr int TI = band_tile<N>();
   const size_t lds = sizeof(float2) * (N + (size_t)N * TI);
-  if (dir < 0) k_bandz_fwd<N><<<nblocks, TI * Plan<N>::TPS, lds, ctx->stream>>>(items, nitems, tw);
-  else k_bandz_inv<N><<<nblocks, TI * Plan<N>::TPS, lds, ctx->stream>>>(items, nitems, tw);
+  constexpr int NT = band_threads<N>();
+  if (dir < 0) k_bandz_fwd<N><<<nblocks, NT, lds, ctx->stream>>>(items, nitems, tw);
+  else k_bandz_inv<N><<<nblocks, NT, lds, ctx->stream>>>(items, nitems, tw);
   return cg::hip_fail(ctx, hipGetLastError(), "k_bandz");
 }
 

@@ -66,10 +66,9 @@ struct BandArgs {
   float2 *band;       // the band's planes [nb][nyp][rnxp] (x forward: in place when band_out is band)
   float2 *band_out;   // x passes: where the rows go
   float *out;         // z inverse: the real grid written
-  const int *kb;      // [nb] the band's frequencies, ascending, 0..nzp/2
   const int *at;      // [nzp/2 + 1] the band's plane of a frequency, or -1
   long rows;          // nb nyp
-  unsigned nb, ncols, cnxp;  // ncols = cnxp nyp float pairs per plane
+  unsigned ncols, cnxp;  // ncols = cnxp nyp float pairs per plane
   int nxp;
   unsigned block0;
   float scale;
