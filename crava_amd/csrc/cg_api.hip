@@ -2757,6 +2757,11 @@ struct cg_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t done = nullptr;
+  // A batch of several inversions is cut into parts of about equal work, each with its own pass
+  // sequence on a side stream of its own; a part (serial) does not fork further.
+  std::vector<cg_batch *> parts;
+  bool serial = false;
+  std::vector<char> host;  // a part's descriptors while their copy is under way
 };
 
 namespace {
@@ -2783,7 +2788,7 @@ template <typename F>
 int fork_join(cg_batch *b, int n, F launch)
 {
   cg_ctx *ctx = b->ctx;
-  if (n < 2 || !ctx->fork) {
+  if (n < 2 || !ctx->fork || b->serial) {
     for (int i = 0; i < n; ++i)
       if (int rc = launch(i)) return rc;
     return CG_OK;
@@ -2832,6 +2837,7 @@ int run_pass(cg_batch *b, const cg_batch::Pass &p)
 void release_batch(cg_batch *b)
 {
   cg_ctx *ctx = b->ctx;
+  for (cg_batch *p : b->parts) release_batch(p);
   (void)hipStreamSynchronize(ctx->stream);  // the side streams join into it
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -2847,6 +2853,7 @@ int enqueue_batch(cg_batch *b)
 {
   cg_ctx *ctx = b->ctx;
   int rc = CG_OK;
+  if (!b->parts.empty()) return fork_join(b, (int)b->parts.size(), [&](int i) { return enqueue_batch(b->parts[i]); });
   if (b->ncounters) rc = cg::zero_counters(ctx, b->counters, b->ncounters);
   for (auto &p : b->fwd)
     if (!rc) rc = run_pass(b, p);
@@ -2874,14 +2881,10 @@ int enqueue_batch(cg_batch *b)
 
 }  // namespace
 
-extern "C" {
+namespace {
 
-int cg_batch_create(cg_ctx *ctx, int n, const cg_inversion *inv, cg_batch **out)
+int validate_batch(cg_ctx *ctx, int n, const cg_inversion *inv)
 {
-  if (!ctx || !inv || !out || n < 1) return CG_EINVAL;
-  *out = nullptr;
-  DeviceGuard dg(ctx->device);
-  // ---- validation
   for (int i = 0; i < n; ++i) {
     const cg_inversion &v = inv[i];
     const cg_post_args &a = v.post;
@@ -2910,6 +2913,64 @@ int cg_batch_create(cg_ctx *ctx, int n, const cg_inversion *inv, cg_batch **out)
     for (int l = 0; l < nt; ++l)
       if (v.seis_in[l]->transformed) return cg::fail(ctx, CG_ESTATE, "batch: inputs must be in the real domain");
   }
+  return CG_OK;
+}
+
+// The inversions of a batch in at most kSide parts of about equal work (largest first, each to the
+// part with the least so far).  Inversions of which one writes a grid that another uses stay in one
+// part: there all forward passes come before the first result is written.
+std::vector<std::vector<int>> batch_parts(int n, const cg_inversion *inv)
+{
+  std::vector<int> root(n);
+  for (int i = 0; i < n; ++i) root[i] = i;
+  auto find = [&](int i) {
+    while (root[i] != i) i = root[i] = root[root[i]];
+    return i;
+  };
+  std::map<const cg_grid *, std::pair<bool, std::vector<int>>> use;  // written by any; users
+  std::vector<double> work(n, 0.0);
+  for (int i = 0; i < n; ++i) {
+    const cg_inversion &v = inv[i];
+    auto add = [&](const cg_grid *g, bool writes) {
+      auto &u = use[g];
+      u.first |= writes;
+      u.second.push_back(i);
+    };
+    for (int g = 0; g < 3; ++g) add(v.mean_in[g], false), add(v.post.mean[g], true);
+    for (int l = 0; l < v.post.ntheta; ++l) add(v.seis_in[l], false), add(v.post.data[l], true);
+    for (int g = 0; g < 6; ++g) add(v.post.cov[g], true);
+    for (int r = 0; r < 3 * v.nreal; ++r) add(v.out[r], true);
+    work[i] = (double)v.mean_in[0]->csize * (8 + v.post.ntheta + 4 * v.nreal);
+  }
+  for (const auto &u : use)
+    if (u.second.first)
+      for (int i : u.second.second) root[find(i)] = find(u.second.second[0]);
+  std::map<int, std::vector<int>> groups;
+  std::map<int, double> weight;
+  for (int i = 0; i < n; ++i) {
+    groups[find(i)].push_back(i);
+    weight[find(i)] += work[i];
+  }
+  std::vector<int> order;
+  for (const auto &g : groups) order.push_back(g.first);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return weight[a] > weight[b]; });
+  std::vector<std::vector<int>> parts(std::min<size_t>(cg_ctx::kSide, order.size()));
+  std::vector<double> load(parts.size(), 0.0);
+  for (int g : order) {
+    const size_t k = std::min_element(load.begin(), load.end()) - load.begin();
+    load[k] += weight[g];
+    parts[k].insert(parts[k].end(), groups[g].begin(), groups[g].end());
+  }
+  for (auto &p : parts) std::sort(p.begin(), p.end());
+  return parts;
+}
+
+// One part of a batch (its copy to the device is left under way), or a batch of one.
+int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch **out)
+{
+  if (!ctx || !inv || !out || n < 1) return CG_EINVAL;
+  *out = nullptr;
+  DeviceGuard dg(ctx->device);
   cg_batch *b = new (std::nothrow) cg_batch();
   if (!b) return CG_ENOMEM;
   b->ctx = ctx;
@@ -3322,12 +3383,59 @@ int cg_batch_create(cg_ctx *ctx, int n, const cg_inversion *inv, cg_batch **out)
     ++gi;
   }
   e = hipMemcpyAsync(b->dev, host.data(), L.size, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
+  if (part) {
+    b->serial = true;
+    b->host = std::move(host);
+  } else {
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
+  }
   if (e == hipSuccess && ensure_side_streams(ctx) != CG_OK) e = hipErrorOutOfMemory;
   if (e != hipSuccess) {
     release_batch(b);
     return cg::hip_fail(ctx, e, "batch: upload of descriptors");
+  }
+  *out = b;
+  return CG_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cg_batch_create(cg_ctx *ctx, int n, const cg_inversion *inv, cg_batch **out)
+{
+  if (!ctx || !inv || !out || n < 1) return CG_EINVAL;
+  *out = nullptr;
+  DeviceGuard dg(ctx->device);
+  if (int rc = validate_batch(ctx, n, inv)) return rc;
+  const auto parts = batch_parts(n, inv);
+  if (parts.size() < 2) return plan_batch(ctx, n, inv, false, out);
+  cg_batch *b = new (std::nothrow) cg_batch();
+  if (!b) return CG_ENOMEM;
+  b->ctx = ctx;
+  b->n = n;
+  b->inv.assign(inv, inv + n);
+  b->outs.resize(n);
+  for (int i = 0; i < n; ++i) {
+    b->outs[i].assign(inv[i].out, inv[i].out + 3 * inv[i].nreal);
+    b->inv[i].out = nullptr;
+  }
+  int rc = CG_OK;
+  for (const auto &p : parts) {
+    std::vector<cg_inversion> sub;
+    for (int i : p) sub.push_back(inv[i]);
+    cg_batch *part = nullptr;
+    rc = plan_batch(ctx, (int)sub.size(), sub.data(), true, &part);
+    if (rc) break;
+    b->parts.push_back(part);
+  }
+  if (!rc) rc = cg::hip_fail(ctx, hipStreamSynchronize(ctx->stream), "batch: upload of descriptors");
+  for (cg_batch *p : b->parts) std::vector<char>().swap(p->host);
+  if (!rc) rc = cg::hip_fail(ctx, hipEventCreateWithFlags(&b->done, hipEventDisableTiming), "batch event");
+  if (rc) {
+    release_batch(b);
+    return rc;
   }
   *out = b;
   return CG_OK;

@@ -1,0 +1,81 @@
+"""A batch of several inversions runs in parts on side streams.  Every inversion equals a batch of
+one bit for bit, with launches and replayed as a graph, for one to six inversions of uneven sizes;
+and inversions that pass grids to each other (one's realisation is another's seismic input, which
+every forward transform reads before a result is written) keep that order."""
+import numpy as np
+import pytest
+
+import crava_amd as C
+import problem as P
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(20, 18, 40), (9, 11, 30), (30, 12, 25), (12, 12, 60), (16, 25, 35), (8, 7, 45)]
+
+
+def _item(ctx, k, nreal):
+    p = P.make_problem(*SIZES[k], seed=100 + k, angles_deg=tuple(np.linspace(0.0, 30.0, 2 + k % 3)))
+    mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    nt = p["ntheta"]
+    it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=k, mean_in=mk(C.PARAMETER, 3),
+              seis_in=mk(C.DATA, nt), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, nt), cov=mk(C.COVARIANCE, 6),
+              out=[mk(C.PARAMETER, 3) for _ in range(nreal)])
+    for g, r in zip(it["mean_in"] + it["seis_in"], list(p["mean_real"]) + list(p["seis_real"])):
+        g.upload_real(r)
+    return it
+
+
+def _results(it):
+    return [g.download_real() for g in it["mean"]] + [g.download_complex() for g in it["cov"]] + \
+           [g.download_real() for r in it["out"] for g in r]
+
+
+def _close(items):
+    for it in items:
+        for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"] + [g for r in it["out"] for g in r]:
+            g.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6])
+def test_parts_equal_batches_of_one(ctx, n):
+    print("parts", n, flush=True)
+    items = [_item(ctx, k, k % 3) for k in range(n)]
+    want = []
+    for it in items:
+        b = C.Batch(ctx, [it])
+        b.run()
+        b.wait()
+        want.append(_results(it))
+        b.close()
+    b = C.Batch(ctx, items)
+    for rep in range(3):
+        if rep == 1:
+            b.use_graph()
+        for it in items:
+            for g in it["mean"] + it["cov"]:
+                g.fillInConstant(-1.0)
+        b.run()
+        b.wait()
+        for it, w in zip(items, want):
+            assert all(np.array_equal(x, y) for x, y in zip(_results(it), w)), (n, rep)
+    b.close()
+    _close(items)
+
+
+def test_grids_handed_on_keep_the_pass_order(ctx):
+    a, c = _item(ctx, 0, 1), _item(ctx, 0, 0)
+    b1 = C.Batch(ctx, [c])
+    b1.run()
+    b1.wait()
+    want = _results(c)
+    b1.close()
+    seis = c["seis_in"][0].download_real(padded=True)
+    a["out"][0][0].setType(C.DATA)  # the realisation grid holds the other's seismic cube first
+    a["out"][0][0].upload_real(seis)
+    shared = dict(c, seis_in=[a["out"][0][0]] + c["seis_in"][1:])
+    b = C.Batch(ctx, [a, shared])
+    b.run()
+    b.wait()
+    assert all(np.array_equal(x, y) for x, y in zip(_results(shared), want))
+    b.close()
+    _close([a, c])
