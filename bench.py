@@ -9,8 +9,8 @@ Workload (one step = one inversion, inputs resident in HBM when the timed region
   the prior and forward-modelled to seismic on the GPU.
   Step: one cg_invert call -- 3 + 5 forward FFTs, per-wavenumber posterior (FP32, FP64 re-solve
   where the pivot ratio of the Cholesky factor exceeds 1e6), 3 inverse FFTs of the posterior
-  means, at this geometry with the z transform split into two stages carried by the x passes and
-  the posterior pass -- then 2 posterior realisations (counter-based noise, colouring, 3 inverse
+  means, at this geometry with the z passes first and last and only the inverted frequencies
+  between them -- then 2 posterior realisations (counter-based noise, colouring, 3 inverse
   FFTs + the real-domain mean each).
 
 Prints one JSON line.  Also reported: per-kernel HIP-event times, the roofline of the dominant
@@ -39,35 +39,29 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def kernel_bytes(w, nt, R, n_inv_planes, launches, split):
+def kernel_bytes(w, nt, R, n_inv_planes):
     """Algorithmic HBM bytes per kernel class for one step (what each kernel must read + write).
-    `launches`: launches per step of each FFT class, as counted on the context stream -- every FFT
-    launch transforms one grid (the realisations' inverse z passes run inside the fused colouring
-    and are not z launches).  split: the request ran the split-z passes (cg_invert) -- the x
-    passes carry the z stages, the posterior pass reads and writes whole grids, and the
-    colouring adds the means in their split layout; otherwise the drop-in sequence (the
-    posterior reads the spectra of inverted planes only, the colouring adds the spectral
-    means).  Either way a pair of realisations reads the means once."""
+    The request runs the band-limited sequence: a forward z pass reads a real cube and writes its
+    inverted frequencies ("band"), the x and y passes and the posterior see the band only, and
+    the inverse z pass adds the update to the prior mean.  The realisations are coloured in pairs
+    with the first inverse z stage, then take a y pass and an x pass that carries the second
+    stage and adds the real-domain mean."""
     G = (w["nxp"] // 2 + 1) * w["nyp"] * w["nzp"] * 8  # one complex grid
     Nr = w["nxp"] * w["nyp"] * w["nzp"] * 4  # one real cube (without row padding)
-    plane = (w["nxp"] // 2 + 1) * w["nyp"]
-    if split:
-        post = (3 + nt + 3 + 6) * G  # z stage 2 needs every plane of the inputs and of the means
-    else:
-        post = n_inv_planes * plane * (3 + nt + 9) * 8 + (w["nzp"] - n_inv_planes) * plane * 6 * 8
+    B = n_inv_planes * (w["nxp"] // 2 + 1) * w["nyp"] * 8  # one grid's band
+    n = 3 + nt
     return {
-        # x: forward reads the real cube and writes the spectrum, inverse the reverse
-        C.K_FFT_X: launches[C.K_FFT_X] * (Nr + G),
-        # y / z: one grid read and written per launch
-        C.K_FFT_Y: launches[C.K_FFT_Y] * 2 * G,
-        C.K_FFT_Z: launches[C.K_FFT_Z] * 2 * G,
-        # split: read 3 + nt grids, write 3 means + 6 covariance grids; drop-in: inverted cells read
-        # 3 + nt spectra and write 3 means + 6 covariance entries, pass-through cells write the 6
-        # prior covariance entries
-        C.K_POSTERIOR: post,
-        # colouring: read 6 covariance and 3 mean spectra, write 3 per realisation (noise
-        # generated in registers); pairs read their inputs once
-        C.K_NOISE: (R // 2) * 15 * G + (R % 2) * 12 * G,
+        # band: every x and y pass reads and writes it; realisations: x reads the spectrum and the
+        # mean and writes the cube, y reads and writes a grid
+        C.K_FFT_X: (n + 3) * 2 * B + 3 * R * (G + 2 * Nr),
+        C.K_FFT_Y: (n + 3) * 2 * B + 3 * R * 2 * G,
+        # forward: cube -> band; inverse: band and prior mean -> mean
+        C.K_FFT_Z: n * (Nr + B) + 3 * (B + 2 * Nr),
+        # reads the band of every input, writes the three updates and the covariance of every plane
+        C.K_POSTERIOR: (n + 3) * B + 6 * G,
+        # colouring: read 6 covariance grids, write 3 per realisation (noise generated in
+        # registers); pairs read their inputs once
+        C.K_NOISE: (R // 2) * 12 * G + (R % 2) * 9 * G,
     }
 
 
@@ -528,9 +522,7 @@ def main():
     for g in inv.out[0]:
         seed = g.fillInComplexNoiseReference(seed)
     ms_refnoise = 1000.0 * (time.perf_counter() - t) / 3
-    split = kt[C.K_FFT_Z][0] == 0  # the split-z request launches no z pass of its own
-    kb = kernel_bytes(w, inv.nt, R, inv.n_inverted_planes,
-                      {k: kt[k][0] // args.profile_steps for k in (C.K_FFT_X, C.K_FFT_Y, C.K_FFT_Z)}, split)
+    kb = kernel_bytes(w, inv.nt, R, inv.n_inverted_planes)
     kernels = {}
     for k, (n, ms) in kt.items():
         if n == 0:

@@ -185,7 +185,7 @@ class Problem:
 
     def step(self, realisations=None, stats=False, precision=PREC_MIXED):
         """One request: cg_invert (forward transforms, posterior, realisations, inverse transforms
-        of the means; the split-z passes where the grid has them).  Realisations beyond the kept
+        of the means; the band-limited or split-z passes where the grid takes them).  Realisations beyond the kept
         output sets are streamed through them afterwards, with the real-domain means.  Returns
         (inverted, failures, FP64 re-solves) when stats (a synchronisation), zeros otherwise."""
         R = self.R if realisations is None else realisations
