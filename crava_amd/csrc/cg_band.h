@@ -157,6 +157,7 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
     const int k = t + i * TPS;
     const int p = first && k <= N / 2 ? at[k] : -1;
     f[i] = p >= 0 ? *(const __attribute__((address_space(1))) fvec4 *)(src + 2 * (size_t)p * a.ncols) : fvec4{0.f, 0.f, 0.f, 0.f};
+    if (!second) f[i].z = f[i].w = 0.f;  // the column past an odd row: the x pass leaves it as the work grid had it
   }
   // the prior mean's pairs of this thread's outputs (element j + r LNB of the column), in flight
   // during the transform

@@ -101,3 +101,27 @@ def test_band_matches_dropin(ctx, name):
         assert rel_l2(b, a) < 5e-6
     for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"] + [g for r in it["out"] for g in r]:
         g.close()
+
+
+@pytest.mark.parametrize("nt", [1, 2, 5])
+def test_work_grid_contents_do_not_matter(ctx, nt):
+    """The outputs and the work grids may hold anything before the call: the results have the same
+    bits after zeros and after NaN.  Odd rows: the columns past the row belong to no pair of traces."""
+    print("work grids", nt, flush=True)
+    p = _problem(nt, (375, 189, 180), high=25.0)
+    mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=5, mean_in=mk(C.PARAMETER, 3),
+              seis_in=mk(C.DATA, nt), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, nt), cov=mk(C.COVARIANCE, 6), out=[])
+    for g, r in zip(it["mean_in"] + it["seis_in"], list(p["mean_real"]) + list(p["seis_real"])):
+        g.upload_real(r)
+    res = []
+    for value in (0.0, np.nan):
+        before = np.full((p["nzp"], p["nyp"], p["nxp"] // 2 + 1), value + 1j * value, np.complex64)
+        for g in it["mean"] + it["data"] + it["cov"]:
+            g.upload_complex(before)
+        C.invert(ctx, it)
+        res.append([g.download_real(padded=True) for g in it["mean"]] + [g.download_complex() for g in it["cov"]])
+    for a, b in zip(*res):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+    for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"]:
+        g.close()
