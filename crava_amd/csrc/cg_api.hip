@@ -4,6 +4,7 @@
 // a device, a HIP stream, a device-memory budget, twiddle tables and staging buffers.  Grids
 // are device-resident in the reference's in-place FFTW layout.
 #include <algorithm>
+#include <array>
 #include <mutex>
 #include <cmath>
 #include <complex>
@@ -2757,10 +2758,9 @@ struct cg_batch {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t done = nullptr;
-  // A batch of several inversions is cut into parts of about equal work, each with its own pass
-  // sequence on a side stream of its own; a part (serial) does not fork further.
+  // A batch of large inversions of several sizes is cut into parts of about equal work
+  // (batch_parts), each with its own pass sequence on a side stream of its own.
   std::vector<cg_batch *> parts;
-  bool serial = false;
   std::vector<char> host;  // a part's descriptors while their copy is under way
 };
 
@@ -2782,13 +2782,13 @@ int ensure_side_streams(cg_ctx *ctx)
   return cg::hip_fail(ctx, e, "side streams");
 }
 
-// Runs launch(i) for i < n: on the context stream when n < 2, else spread over the side streams
-// between a fork from and a join into the context stream.
+// Runs launch(i) for i < n: spread over the side streams between a fork from and a join into the
+// context stream, or (fork false, or a single launch) one after the other on the context stream.
 template <typename F>
-int fork_join(cg_batch *b, int n, F launch)
+int fork_join(cg_batch *b, bool fork, int n, F launch)
 {
   cg_ctx *ctx = b->ctx;
-  if (n < 2 || !ctx->fork || b->serial) {
+  if (n < 2 || !ctx->fork || !fork) {
     for (int i = 0; i < n; ++i)
       if (int rc = launch(i)) return rc;
     return CG_OK;
@@ -2812,10 +2812,10 @@ int fork_join(cg_batch *b, int n, F launch)
   return cg::hip_fail(ctx, e, "batch join");
 }
 
-int run_pass(cg_batch *b, const cg_batch::Pass &p)
+int run_pass(cg_batch *b, bool fork, const cg_batch::Pass &p)
 {
   cg_ctx *ctx = b->ctx;
-  int rc = fork_join(b, (int)p.fixed.size(), [&](int i) {
+  int rc = fork_join(b, fork, (int)p.fixed.size(), [&](int i) {
     const auto &g = p.fixed[i];
     hipEvent_t ev;
     cg::launch_begin(ctx, p.kclass, &ev);
@@ -2849,32 +2849,34 @@ void release_batch(cg_batch *b)
   delete b;
 }
 
-int enqueue_batch(cg_batch *b)
+// fork: the launches of each pass of a batch without parts run side by side.
+int enqueue_batch(cg_batch *b, bool fork)
 {
   cg_ctx *ctx = b->ctx;
   int rc = CG_OK;
-  if (!b->parts.empty()) return fork_join(b, (int)b->parts.size(), [&](int i) { return enqueue_batch(b->parts[i]); });
+  if (!b->parts.empty())
+    return fork_join(b, true, (int)b->parts.size(), [&](int i) { return enqueue_batch(b->parts[i], false); });
   if (b->ncounters) rc = cg::zero_counters(ctx, b->counters, b->ncounters);
   for (auto &p : b->fwd)
-    if (!rc) rc = run_pass(b, p);
+    if (!rc) rc = run_pass(b, fork, p);
   if (!rc)
-    rc = fork_join(b, (int)b->post.size(), [&](int i) {
+    rc = fork_join(b, fork, (int)b->post.size(), [&](int i) {
       const auto &g = b->post[i];
       return cg::launch_posterior_batch(ctx, g.nt, g.sep, g.mixed, g.items, g.nitems, g.blocks);
     });
   for (auto &p : b->inv_mean)
-    if (!rc) rc = run_pass(b, p);
+    if (!rc) rc = run_pass(b, fork, p);
   for (size_t r = 0; r < b->sim.size(); ++r) {
     const auto &cp = b->colour[r];
     if (!rc)
-      rc = fork_join(b, 1 + (int)cp.fused.size(), [&](int k) {
+      rc = fork_join(b, fork, 1 + (int)cp.fused.size(), [&](int k) {
         if (k == 0) return cg::colour_batch(ctx, cp.items, cp.nitems, cp.blocks);
         const auto &f = cp.fused[k - 1];
         return f.pair ? cg::fixed_colour_zinv2_list(ctx, f.e, f.items, f.nitems, f.blocks)
                       : cg::fixed_colour_zinv_list(ctx, f.e, f.items, f.nitems, f.blocks);
       });
     for (auto &p : b->sim[r])
-      if (!rc) rc = run_pass(b, p);
+      if (!rc) rc = run_pass(b, fork, p);
   }
   return rc;
 }
@@ -2917,55 +2919,44 @@ int validate_batch(cg_ctx *ctx, int n, const cg_inversion *inv)
 }
 
 // The inversions of a batch in at most kSide parts of about equal work (largest first, each to the
-// part with the least so far).  Inversions of which one writes a grid that another uses stay in one
-// part: there all forward passes come before the first result is written.
+// part with the least so far).  Inversions of one padded geometry stay in one part: they share every
+// launch, and only they can hand grids to each other (there all forward passes come before the
+// first result is written).  Four cubes of 84 x 84 x 180 replayed as a graph: 310 us together, 330 in
+// four parts; of 48 x 48 x 96: 88 and 193.  Small cubes stay together whatever their sizes: a part's
+// launches are then shorter than what the streams cost (microseconds per replay, in parts / together:
+// sixteen cubes of 65 thousand cells on average 405 / 224, of 203 652 / 503, four of 65 191 / 116, of 205
+// 232 / 227; sixteen of 306 427 / 435, of 700 778 / 803, two of 570 116 / 136, four of 890 238 / 287).
+constexpr double kPartCells = 1 << 18;
 std::vector<std::vector<int>> batch_parts(int n, const cg_inversion *inv)
 {
-  std::vector<int> root(n);
-  for (int i = 0; i < n; ++i) root[i] = i;
-  auto find = [&](int i) {
-    while (root[i] != i) i = root[i] = root[root[i]];
-    return i;
+  struct Group {
+    std::vector<int> of;
+    double work = 0.0;
   };
-  std::map<const cg_grid *, std::pair<bool, std::vector<int>>> use;  // written by any; users
-  std::vector<double> work(n, 0.0);
+  std::map<std::array<int, 3>, Group> geometries;
+  double cells = 0.0;
   for (int i = 0; i < n; ++i) {
-    const cg_inversion &v = inv[i];
-    auto add = [&](const cg_grid *g, bool writes) {
-      auto &u = use[g];
-      u.first |= writes;
-      u.second.push_back(i);
-    };
-    for (int g = 0; g < 3; ++g) add(v.mean_in[g], false), add(v.post.mean[g], true);
-    for (int l = 0; l < v.post.ntheta; ++l) add(v.seis_in[l], false), add(v.post.data[l], true);
-    for (int g = 0; g < 6; ++g) add(v.post.cov[g], true);
-    for (int r = 0; r < 3 * v.nreal; ++r) add(v.out[r], true);
-    work[i] = (double)v.mean_in[0]->csize * (8 + v.post.ntheta + 4 * v.nreal);
+    const cg_grid *g = inv[i].mean_in[0];
+    Group &q = geometries[{g->nxp, g->nyp, g->nzp}];
+    q.of.push_back(i);
+    q.work += (double)g->csize * (8 + inv[i].post.ntheta + 4 * inv[i].nreal);
+    cells += (double)g->nxp * g->nyp * g->nzp;
   }
-  for (const auto &u : use)
-    if (u.second.first)
-      for (int i : u.second.second) root[find(i)] = find(u.second.second[0]);
-  std::map<int, std::vector<int>> groups;
-  std::map<int, double> weight;
-  for (int i = 0; i < n; ++i) {
-    groups[find(i)].push_back(i);
-    weight[find(i)] += work[i];
-  }
-  std::vector<int> order;
-  for (const auto &g : groups) order.push_back(g.first);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return weight[a] > weight[b]; });
-  std::vector<std::vector<int>> parts(std::min<size_t>(cg_ctx::kSide, order.size()));
+  std::vector<const Group *> order;
+  for (const auto &g : geometries) order.push_back(&g.second);
+  std::stable_sort(order.begin(), order.end(), [](const Group *a, const Group *b) { return a->work > b->work; });
+  std::vector<std::vector<int>> parts(cells < n * kPartCells ? 1 : std::min<size_t>(cg_ctx::kSide, order.size()));
   std::vector<double> load(parts.size(), 0.0);
-  for (int g : order) {
+  for (const Group *g : order) {
     const size_t k = std::min_element(load.begin(), load.end()) - load.begin();
-    load[k] += weight[g];
-    parts[k].insert(parts[k].end(), groups[g].begin(), groups[g].end());
+    load[k] += g->work;
+    parts[k].insert(parts[k].end(), g->of.begin(), g->of.end());
   }
   for (auto &p : parts) std::sort(p.begin(), p.end());
   return parts;
 }
 
-// One part of a batch (its copy to the device is left under way), or a batch of one.
+// One part of a batch (its copy to the device is left under way), or a whole one.
 int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch **out)
 {
   if (!ctx || !inv || !out || n < 1) return CG_EINVAL;
@@ -3384,7 +3375,6 @@ int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch 
   }
   e = hipMemcpyAsync(b->dev, host.data(), L.size, hipMemcpyHostToDevice, ctx->stream);
   if (part) {
-    b->serial = true;
     b->host = std::move(host);
   } else {
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -3448,6 +3438,13 @@ int cg_batch_use_graph(cg_batch *b, int enable)
   return CG_OK;
 }
 
+// Inversions from which the passes of a captured batch without parts fork: in a replayed graph a fork
+// costs about what the overlap of a few small launches gives (small cubes of different sizes with a
+// realisation, one after the other / forked: two 115 / 125 us, four 201 / 192, eight 314 / 264, sixteen
+// 444 / 322).  Launched one by one, without a graph, the forks' events cost the host more than the
+// launches: eight 307 / 892 us.
+constexpr int kForkFrom = 6;
+
 int cg_batch_run(cg_batch *b)
 {
   if (!b) return CG_EINVAL;
@@ -3463,7 +3460,7 @@ int cg_batch_run(cg_batch *b)
         ctx->profiling = prof;
         return cg::hip_fail(ctx, e, "hipStreamBeginCapture");
       }
-      rc = enqueue_batch(b);
+      rc = enqueue_batch(b, b->n >= kForkFrom);
       e = hipStreamEndCapture(ctx->stream, &b->graph);
       ctx->profiling = prof;
       if (rc) return rc;
@@ -3472,7 +3469,7 @@ int cg_batch_run(cg_batch *b)
     }
     rc = cg::hip_fail(ctx, hipGraphLaunch(b->exec, ctx->stream), "hipGraphLaunch");
   } else {
-    rc = enqueue_batch(b);
+    rc = enqueue_batch(b, false);
   }
   if (rc) return rc;
   for (int i = 0; i < b->n; ++i) {  // domains after a run

@@ -416,9 +416,11 @@ int cg_grid_fill_noise_reference(cg_grid *grid, uint32_t *seed);
 
 /* ------------------------------------------------------------------ batched inversions */
 /* Many independent inversions of any sizes (the reference runs one per process) planned
- * together: each pass of all of them shares a few launches (one per compiled FFT length, run
- * concurrently on side streams; one posterior launch per angle count; colouring), so small
- * cubes no longer pay one launch per grid and pass.  No reference counterpart; it serves
+ * together, so that small cubes no longer pay one launch per grid and pass: a pass of several
+ * inversions shares a few launches (one per compiled FFT length; one posterior launch per angle
+ * count; colouring).  Small inversions, and inversions of one padded size, all share them; a batch
+ * of larger ones of several sizes is cut into up to four parts that run side by side, each with
+ * launches of its own.  No reference counterpart; it serves
  * batched and continuously batched requests.  Results are identical to running each inversion
  * alone in a batch of one.  Grids may belong to any context on the same device (a server
  * generates inputs on one stream and runs batches on others); the batch runs on the stream of

@@ -1,4 +1,5 @@
-"""A batch of several inversions runs in parts on side streams.  Every inversion equals a batch of
+"""A batch of several larger inversions runs in parts on side streams, small ones and ones of equal
+size share their launches.  Every inversion equals a batch of
 one bit for bit, with launches and replayed as a graph, for one to six inversions of uneven sizes;
 and inversions that pass grids to each other (one's realisation is another's seismic input, which
 every forward transform reads before a result is written) keep that order."""
@@ -13,8 +14,8 @@ pytestmark = pytest.mark.gpu
 SIZES = [(20, 18, 40), (9, 11, 30), (30, 12, 25), (12, 12, 60), (16, 25, 35), (8, 7, 45)]
 
 
-def _item(ctx, k, nreal):
-    p = P.make_problem(*SIZES[k], seed=100 + k, angles_deg=tuple(np.linspace(0.0, 30.0, 2 + k % 3)))
+def _item(ctx, k, nreal, sizes=SIZES):
+    p = P.make_problem(*sizes[k], seed=100 + k, angles_deg=tuple(np.linspace(0.0, 30.0, 2 + k % 3)))
     mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
     nt = p["ntheta"]
     it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=k, mean_in=mk(C.PARAMETER, 3),
@@ -79,3 +80,45 @@ def test_grids_handed_on_keep_the_pass_order(ctx):
     assert all(np.array_equal(x, y) for x, y in zip(_results(shared), want))
     b.close()
     _close([a, c])
+
+
+LARGE = [(70, 60, 80), (75, 48, 100), (60, 80, 70), (72, 64, 90), (70, 60, 80)]  # over 2^18 padded cells each
+
+
+@pytest.mark.parametrize("sizes", [LARGE[:2], LARGE, LARGE[:1] * 3, SIZES[:2], SIZES, SIZES[:1] * 4],
+                         ids=["large two", "large five", "large equal", "small two", "small six", "small equal"])
+def test_shared_launches(ctx, sizes):
+    """x launches of a run: together, each pass (forward, means, realisations) has one per row length;
+    parts have their own.  The results are those of batches of one either way."""
+    print("launches", sizes, flush=True)
+    items = [_item(ctx, k, 1, sizes) for k in range(len(sizes))]
+    want = []
+    for it in items:
+        b = C.Batch(ctx, [it])
+        b.run()
+        b.wait()
+        want.append(_results(it))
+        b.close()
+    b = C.Batch(ctx, items)
+    ctx.set_profiling(True)
+    ctx.reset_kernel_time()
+    b.run()
+    b.wait()
+    launches = ctx.kernel_time(C.K_FFT_X)[0]
+    ctx.set_profiling(False)
+    got = [_results(it) for it in items]
+    b.use_graph()
+    b.run()
+    b.wait()
+    for it, w, g in zip(items, want, got):
+        assert all(np.array_equal(x, y) for x, y in zip(g, w))
+        assert all(np.array_equal(x, y) for x, y in zip(_results(it), w))
+    lengths = len({it["mean"][0].nxp for it in items})
+    geometries = len({(it["mean"][0].nxp, it["mean"][0].nyp, it["mean"][0].nzp) for it in items})
+    print("%d inversions, %d geometries, %d row lengths: %d x launches" % (len(items), geometries, lengths, launches))
+    if sizes[0] in LARGE and geometries > 1:
+        assert launches == 3 * geometries  # at most four geometries: a part each
+    else:
+        assert launches == 3 * lengths
+    b.close()
+    _close(items)
