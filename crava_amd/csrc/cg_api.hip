@@ -3421,7 +3421,8 @@ int cg_batch_create(cg_ctx *ctx, int n, const cg_inversion *inv, cg_batch **out)
     b->parts.push_back(part);
   }
   if (!rc) rc = cg::hip_fail(ctx, hipStreamSynchronize(ctx->stream), "batch: upload of descriptors");
-  for (cg_batch *p : b->parts) std::vector<char>().swap(p->host);
+  if (!rc)  // on an error release_batch waits for the copies before it frees what they read
+    for (cg_batch *p : b->parts) std::vector<char>().swap(p->host);
   if (!rc) rc = cg::hip_fail(ctx, hipEventCreateWithFlags(&b->done, hipEventDisableTiming), "batch event");
   if (rc) {
     release_batch(b);

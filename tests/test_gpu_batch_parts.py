@@ -122,3 +122,32 @@ def test_shared_launches(ctx, sizes):
         assert launches == 3 * lengths
     b.close()
     _close(items)
+
+
+def test_a_part_that_cannot_be_planned(ctx):
+    """The second part's z axis is too long for a workgroup's LDS: the batch is refused, what the first
+    part held is given back once its copy to the device is over, and other batches run as before."""
+    good = _item(ctx, 0, 0, LARGE)
+    p = P.make_problem(2, 2, 50, nxp=4, nyp=4, nzp=64, angles_deg=(0.0,))
+    for name in ("K", "e1", "e2", "e3", "invert", "rt"):
+        p[name] = np.resize(p[name], (7000,) + p[name].shape[1:])
+    p.update(nz=6000, nzp=7000)
+    mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    bad = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=1, mean_in=mk(C.PARAMETER, 3),
+               seis_in=mk(C.DATA, 1), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, 1), cov=mk(C.COVARIANCE, 6), out=[])
+    b = C.Batch(ctx, [good])
+    b.run()
+    b.wait()
+    want = _results(good)
+    b.close()
+    held = ctx.memory()[0]
+    for _ in range(3):
+        with pytest.raises(C.CravaError, match="too long"):
+            C.Batch(ctx, [good, bad])
+        assert ctx.memory()[0] == held
+    b = C.Batch(ctx, [good])
+    b.run()
+    b.wait()
+    assert all(np.array_equal(x, y) for x, y in zip(_results(good), want))
+    b.close()
+    _close([good, bad])
