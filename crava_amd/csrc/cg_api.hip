@@ -1201,10 +1201,11 @@ static int post_stats(cg_ctx *ctx, const unsigned long long *dev_counters, bool 
 // Stages the tables of a posterior call (and `extra`, whose device addresses follow them in dp) in
 // one copy, makes room for the FP64 deferral list, clears the counters and fills p.
 // placed, if given, is told the addresses and the index of the first extra part before the copy, so
-// that parts may hold addresses of others.
+// that parts may hold addresses of others.  own_list, if given, is room for the deferral list.
 static int post_stage(cg_ctx *ctx, const cg_post_args *a, const std::vector<std::pair<const void *, size_t>> &extra,
                       std::vector<void *> &dp, cg::PostParams &p,
-                      const std::function<void(const std::vector<void *> &, size_t)> &placed = nullptr)
+                      const std::function<void(const std::vector<void *> &, size_t)> &placed = nullptr,
+                      unsigned *own_list = nullptr)
 {
   const cg_grid *ref = a->mean[0];
   const int nyp = ref->nyp, nzp = ref->nzp, cnxp = ref->cnxp;
@@ -1231,8 +1232,8 @@ static int post_stage(cg_ctx *ctx, const cg_post_args *a, const std::vector<std:
   int rc = stage_tables(ctx, parts, dp, placed ? [&](const std::vector<void *> &d) { placed(d, 6); }
                                                : std::function<void(const std::vector<void *> &)>());
   if (rc) return rc;
-  unsigned *list = nullptr;
-  if (mixed) {
+  unsigned *list = mixed ? own_list : nullptr;
+  if (mixed && !list) {
     if (ctx->list_bytes < list_bytes) {
       (void)hipStreamSynchronize(ctx->stream);
       if (ctx->list) {
@@ -1538,6 +1539,28 @@ constexpr double kBandMost = 0.75, kBandMostSplit = 0.62;
 // Bytes of the band planes one launch of it covers.
 constexpr size_t kBandChunk = (size_t)96 << 20;
 
+// Marks the work grids of an inversion as the transformed inputs, as the drop-in calls would leave
+// them, until restore() takes it back.
+struct WorkMarks {
+  std::vector<cg_grid *> work;
+  std::vector<std::pair<int, int>> before;
+  WorkMarks(const std::vector<cg_grid *> &w, const std::vector<const cg_grid *> &in) : work(w)
+  {
+    for (size_t i = 0; i < work.size(); ++i) {
+      before.push_back({work[i]->cubetype, work[i]->transformed});
+      work[i]->cubetype = in[i]->cubetype;
+      work[i]->transformed = 1;
+    }
+  }
+  void restore()
+  {
+    for (size_t i = 0; i < work.size(); ++i) {
+      work[i]->cubetype = before[i].first;
+      work[i]->transformed = before[i].second;
+    }
+  }
+};
+
 struct GridPasses {
   const cg::FixedEntry *x = nullptr, *y = nullptr, *z = nullptr;
   const cg_grid *ref = nullptr;
@@ -1688,17 +1711,9 @@ static int invert_band(cg_ctx *ctx, const cg_inversion *v)
   distinct.insert(in.begin(), in.end());
   distinct.insert(a.cov, a.cov + 6);
   if (distinct.size() != 2 * work.size() + 6) return 1;
-  std::vector<std::pair<int, int>> before;
-  for (size_t i = 0; i < work.size(); ++i) {
-    before.push_back({work[i]->cubetype, work[i]->transformed});
-    work[i]->cubetype = in[i]->cubetype;
-    work[i]->transformed = 1;
-  }
+  WorkMarks marks(work, in);
   if (post_validate(ctx, &a)) {  // the drop-in calls refuse it
-    for (size_t i = 0; i < work.size(); ++i) {
-      work[i]->cubetype = before[i].first;
-      work[i]->transformed = before[i].second;
-    }
+    marks.restore();
     return 1;
   }
   // descriptors: one per grid and pass, the launches take runs of `chunk` of them
@@ -1741,13 +1756,24 @@ static int invert_band(cg_ctx *ctx, const cg_inversion *v)
   std::vector<std::pair<const void *, size_t>> extra = {{at.data(), sizeof(int) * at.size()}};
   for (const auto *l : {&zf, &xf, &xi, &zi}) extra.push_back({l->data(), sizeof(cg::BandArgs) * l->size()});
   for (const auto *l : {&yf, &yi}) extra.push_back({l->data(), sizeof(cg::StridedArgs) * l->size()});
+  // The FP64 deferral list lies in the first mean's work grid past its band, which nothing uses before
+  // the last z pass, wherever it fits (bands of up to two thirds of the planes, so on every split-z
+  // geometry): those held a list of tiles, 1 MB at 1152 x 1152 x 384 where this one takes 409 MB.
+  size_t ninv = 0;
+  for (int k = 0; k < nzp; ++k) ninv += a.invert[k] != 0;
+  unsigned *list = ninv * plane * sizeof(unsigned) <= (ref->csize - cells) * sizeof(float2)
+                       ? reinterpret_cast<unsigned *>(reinterpret_cast<float2 *>(a.mean[0]->d) + cells)
+                       : nullptr;
   std::vector<void *> dp;
   cg::PostBandArgs pb;
   int rc = post_stage(ctx, &a, extra, dp, pb.p, [&](const std::vector<void *> &d, size_t first) {
     for (auto *l : {&zf, &xf, &xi, &zi})
       for (auto &b : *l) b.at = static_cast<const int *>(d[first]);
-  });
-  if (rc) return rc;
+  }, list);
+  if (rc) {
+    marks.restore();
+    return rc;
+  }
   const size_t e0 = dp.size() - extra.size();
   pb.at = static_cast<const int *>(dp[e0]);
   pb.by_cnxp = cg::make_fastdiv((uint32_t)cnxp);
@@ -1807,17 +1833,9 @@ static int invert_lists(cg_ctx *ctx, const cg_inversion *v)
   distinct.insert(in.begin(), in.end());
   distinct.insert(v->out, v->out + 3 * v->nreal);
   if (distinct.size() != 2 * work.size() + 3 * (size_t)v->nreal) return 1;
-  std::vector<std::pair<int, int>> before;
-  for (size_t i = 0; i < work.size(); ++i) {
-    before.push_back({work[i]->cubetype, work[i]->transformed});
-    work[i]->cubetype = in[i]->cubetype;
-    work[i]->transformed = 1;
-  }
-  if (post_validate(ctx, &a)) {
-    for (size_t i = 0; i < work.size(); ++i) {
-      work[i]->cubetype = before[i].first;
-      work[i]->transformed = before[i].second;
-    }
+  WorkMarks marks(work, in);
+  if (post_validate(ctx, &a)) {  // the drop-in calls refuse it
+    marks.restore();
     return 1;
   }
   // the scales of grid_fft_forward / grid_fft_inverse
@@ -1861,7 +1879,10 @@ static int invert_lists(cg_ctx *ctx, const cg_inversion *v)
   std::vector<void *> dp;
   cg::PostParams p;
   int rc = post_stage(ctx, &a, extra, dp, p);
-  if (rc) return rc;
+  if (rc) {
+    marks.restore();
+    return rc;
+  }
   gp.dev = &dp;
   gp.dev0 = dp.size() - extra.size();
   rc = gp.run(ctx, 0, n_fwd);

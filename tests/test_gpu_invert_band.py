@@ -29,6 +29,8 @@ CASES = {
     "self-mirrored planes": dict(shape=(252, 240, 210), nt=3, planes=(0, 105, 1, 209, 30, 180)),
     "one-sided planes": dict(shape=(250, 245, 200), nt=3, planes=(20, 21, 190, 100)),
     "re-solves": dict(shape=(256, 250, 200), nt=5, sn=1e8),
+    # 72% of the planes: the FP64 list does not fit past the band in a work grid
+    "re-solves, wide band": dict(shape=(256, 250, 200), nt=5, sn=1e8, few=4, planes=tuple(range(1, 73)) + tuple(range(128, 200))),
     "failures": dict(shape=(240, 250, 210), nt=3, precision=C.PREC_REFERENCE, fail=True),
 }
 
@@ -82,7 +84,7 @@ def test_band_matches_dropin(ctx, name):
     (m0, c0, o0, s0, _), (m1, c1, o1, s1, z1) = res[C.FFT_GENERIC], res[C.FFT_AUTO]
     assert s1 == s0
     if kw.get("sn"):
-        assert s1[2] > s1[0] // 2
+        assert s1[2] > s1[0] // kw.get("few", 2)  # the wide band's outer planes are well conditioned
     if kw.get("fail"):
         assert s1[0] == s1[1] > 0
     assert all(np.array_equal(a, b) for a, b in zip(c0, c1))
@@ -125,3 +127,22 @@ def test_work_grid_contents_do_not_matter(ctx, nt):
         assert np.all(np.isfinite(a)) and np.array_equal(a, b)
     for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"]:
         g.close()
+
+
+def test_deferral_list_needs_no_memory():
+    """On the split-z geometries a call holds no list of 4 bytes per inverted wavenumber (11 MB here, 409 MB
+    at 1152 x 1152 x 384): a budget for the grids and 4 MB more takes another grid after it."""
+    nt, shape = 5, (576, 72, 320)
+    p = _problem(nt, shape, sn=1e8)
+    dims = (p["nx"], p["ny"], p["nz"], *shape)
+    grid = C.lib().cg_arena_grid_bytes(*shape)
+    with C.Context(0, hbm_budget=23 * grid + (4 << 20)) as own:
+        mk = lambda ct, n: [C.FFTGrid(own, *dims, ct) for _ in range(n)]
+        it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=5, mean_in=mk(C.PARAMETER, 3),
+                  seis_in=mk(C.DATA, nt), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, nt), cov=mk(C.COVARIANCE, 6), out=[])
+        for g, r in zip(it["mean_in"] + it["seis_in"], list(p["mean_real"]) + list(p["seis_real"])):
+            g.upload_real(r)
+        stats = C.invert(own, it, stats=True)
+        print("deferral list", stats, own.memory(), 22 * grid, flush=True)
+        assert stats[2] > stats[0] // 2
+        C.FFTGrid(own, *dims, C.DATA).close()
