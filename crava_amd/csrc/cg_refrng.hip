@@ -413,11 +413,13 @@ __device__ inline long long draws_before(long i, int cnxp, int nyp, int nzp, con
   return rowbase[jk] + d0 + 2ll * (xs - 1);
 }
 
+// status as k_chain sets it: a stream that does not hold the normals leaves the grid alone.
 __global__ void k_noise_cells(float2 *__restrict__ out, long csize, int cnxp, int nyp, int nzp,
-                              const long long *__restrict__ rowbase, const double *__restrict__ X)
+                              const long long *__restrict__ rowbase, const double *__restrict__ X,
+                              const unsigned long long *__restrict__ status)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= csize) return;
+  if (i >= csize || *status != 0) return;
   const double sd = (double)(float)(1.0 / sqrt(2.0));  // fftgrid.cpp:1003, a float
   long src = i;
   bool conj = false, self = false;
@@ -500,6 +502,10 @@ int fill_noise_reference(cg_ctx *ctx, float2 *out, int nxp, int nyp, int nzp, ui
   double *X = reinterpret_cast<double *>(dev + o_x);
   unsigned long long *end_pos = reinterpret_cast<unsigned long long *>(dev + o_end);
   e = hipMemcpyAsync(rowbase_d, rowbase.data(), sizeof(long long) * (rows + 1), hipMemcpyHostToDevice, ctx->stream);
+  if (e != hipSuccess) {  // nothing may be launched on row bases that did not arrive
+    dev_free(ctx, dev);
+    return hip_fail(ctx, e, "reference noise: upload");
+  }
   auto blocks = [](long n) { return (unsigned)((n + kThreads - 1) / kThreads); };
   hipEvent_t ev;
   launch_begin(ctx, CG_K_NOISE, &ev);
@@ -508,10 +514,11 @@ int fill_noise_reference(cg_ctx *ctx, float2 *out, int nxp, int nyp, int nzp, ui
   k_chain<<<1, kThreadsRng, 0, ctx->stream>>>(s0, nchunks, ngroups, maps, gmaps, nnorm, gentry, gfirst, end_pos + 1);
   k_chunk_entries<<<(unsigned)ngroups, kThreadsRng, 0, ctx->stream>>>(s0, nchunks, maps, gentry, gfirst, centry, cfirst);
   k_emit<<<(unsigned)nchunks, 64, 0, ctx->stream>>>(s0, centry, cfirst, nnorm, X, end_pos);
-  k_noise_cells<<<blocks(csize), kThreads, 0, ctx->stream>>>(out, csize, cnxp, nyp, nzp, rowbase_d, X);
+  k_noise_cells<<<blocks(csize), kThreads, 0, ctx->stream>>>(out, csize, cnxp, nyp, nzp, rowbase_d, X,
+                                                                end_pos + 1);
   launch_end(ctx, CG_K_NOISE, ev);
   unsigned long long got[2] = {0, 0};  // end offset, status
-  if (e == hipSuccess) e = hipGetLastError();
+  e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(got, end_pos, sizeof(got), hipMemcpyDeviceToHost, ctx->stream);
   const hipError_t es = hipStreamSynchronize(ctx->stream);
   dev_free(ctx, dev);
