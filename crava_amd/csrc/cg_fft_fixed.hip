@@ -110,7 +110,7 @@ int fixed_x(cg_ctx *ctx, int forward, const float *src, float *grid, int nxp, lo
   // whose smallest spectral values are the rounding of these transforms, the solve follows every bit
   // of them (the residual of a 280 x 270 x 243 posterior moves by 8e-6 where its own error is 4e-5).
   int v = fixed_variant(ctx, e, rows, forward, add != nullptr);
-  if (v == 0 && even && forward) v = 2;
+  if (v == 0 && even && forward && ctx->fft_variant < 0) v = 2;  // a forced variant is taken as it is
   const unsigned long nblk = ((unsigned long)rows + e->tile[v] - 1) / e->tile[v];
   if (nblk >= (1ul << 31)) {
     *rc = fail(ctx, CG_EINVAL, "x FFT: too many rows");

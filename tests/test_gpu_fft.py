@@ -147,10 +147,11 @@ def _factorable(n):
 PLAN_LENGTHS = [n for n in range(2, 1153) if _factorable(n)]
 
 
-@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("variant", [0, 1, -1])
 def test_every_compiled_length_matches_oracle(ctx, variant):
     """y and z passes of every length, x passes of every even nxp = 2n (n <= 576) and every odd
-    nxp = n, in both tile variants: forward and inverse against the FP64 oracle."""
+    nxp = n, in both tile variants and in the one that runs unasked (even rows forward take a kernel of
+    their own then): forward and inverse against the FP64 oracle."""
     ctx.set_fft_variant(variant)
     rng = np.random.default_rng(11 + variant)
     shapes = []
@@ -181,7 +182,7 @@ def test_every_compiled_length_matches_oracle(ctx, variant):
     print("compiled lengths, variant %d: %d grids, worst rel L2 %.2e" % (variant, len(shapes), worst), flush=True)
 
 
-@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("variant", [0, 1, -1])
 def test_x_pass_tails_and_multi_tile_walks(ctx, variant):
     """Even-nxp x passes on row counts that leave a partial last tile with an odd number of rows
     (the double-buffered kernel copies an odd float2 count, its last element by a plain load),
