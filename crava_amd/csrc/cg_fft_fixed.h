@@ -504,7 +504,9 @@ k_fftx_c2r(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const
 //   nxp 280, 270 x 243 rows   38.3 / 37.4  39.9 / 35.2 52.4 / 48.7 4.0-4.6
 //   nxp 224, 280 x 200 rows   30.4 / 26.6  33.5 / 25.2 42.0 / 36.7 3.8-4.1
 //   nxp 84,  84 x 180 rows     7.4 / 4.3    8.9 / 4.7  10.1 / 5.1  2.2-3.1
-// Memory bounds it at the long lengths (128-byte stores at rows' odd pitch), latency at the short.
+// (the forward rows of nxp 84 and 224 before they were staged, see Row: four grids of 224 in a launch 95 ->
+// 79 us since).  Memory bounds it at the long lengths (128-byte stores at rows' odd pitch), latency at
+// the short.
 constexpr int row_split(int n)  // P1 (<= P2 = n / P1): the factors closest to sqrt(n); 0: none
 {
   int best = 0;
@@ -516,14 +518,27 @@ constexpr int row_split(int n)  // P1 (<= P2 = n / P1): the factors closest to s
 template <int N>
 struct Row {
   static constexpr int P1 = row_split(N);
-  static constexpr bool OK = P1 > 0;
-  static constexpr int P2 = OK ? N / (OK ? P1 : 1) : 1;
+  static constexpr int P2 = P1 > 0 ? N / (P1 > 0 ? P1 : 1) : 1;
+  // Not where the second stage has less than a quarter of the lanes: 5 x 25 alone of the lengths (nxp
+  // 250; the plan's kernel / this one, 4 or 3 grids of 45 MB: forward 91 / 151 us, inverse 82 / 95, inverse +
+  // add 113 / 178).  The single-radix lengths are latency-bound, and faster here.
+  static constexpr bool OK = P1 > 0 && (P2 <= 4 * P1 || P1 == 1);
+  // Rows that leave through LDS as one span of memory: else every lane group of P1 stores segments of
+  // 8 P1 bytes.  Forward below 80 bytes, inverse + add where the second stage has at most half of the lanes
+  // (direct / staged, grids of 45 MB, plan's kernel in brackets: forward 5 x 10 96 / 65 us (76), 7 x 14 88 / 71
+  // (74), 8 x 16 80 / 66 (69), 3 x 9 119 / 79 (86); inverse + add 5 x 15 115 / 75 us (98), 7 x 14 96 / 77 (72),
+  // 9 x 27 127 / 90 (106), 10 x 25 121 / 87 (102)).  Elsewhere direct stores are as fast or faster, up to 1.2
+  // times on grids in the cache (inverse, whose lines the loads have brought there, at every length).
+  static constexpr bool STAGE_FWD = P1 < 10, STAGE_ADD = P2 >= 2 * P1;
   static constexpr int T = P2;           // lanes per sequence
   static constexpr int R = 64 / T;       // sequences per wavefront
   static constexpr int WAVES = 4;        // wavefronts per workgroup
   static constexpr int SEQS = WAVES * R;
   static constexpr int PITCH = P2 | 1;
-  static constexpr int LDS = R * P1 * PITCH;  // float2 per wavefront
+  static constexpr int lds(bool staged)  // float2 per wavefront
+  {
+    return R * (staged && P1 * PITCH < N + 1 ? N + 1 : P1 * PITCH);
+  }
 };
 
 // Keeps the compiler from moving LDS accesses across the exchange.  The hardware needs nothing:
@@ -584,8 +599,9 @@ k_rowe(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const flo
 {
   using P = Row<N>;
   constexpr int P1 = P::P1, P2 = P::P2, CN = N + 1;
+  constexpr bool STAGED = FWD ? P::STAGE_FWD : ADD && P::STAGE_ADD;
   __shared__ float2 tw[2 * N];
-  __shared__ float2 lds[P::WAVES][P::LDS];
+  __shared__ float2 lds[P::WAVES][P::lds(STAGED)];
   cg::XArgs a;
   const unsigned blk = resolve(one, items, nitems, a);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -603,22 +619,46 @@ k_rowe(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const flo
   load_tw(tw, tw_row, 2 * N, tid, 64 * P::WAVES);
   lds_sync();
   float2 *buf = lds[tid >> 6] + (r < P::R ? r : 0) * P1 * P::PITCH;
+  // the wavefront's rows are one span of memory: staged, element i leaves from lane i % 64
+  float2 *const span = lds[tid >> 6];
+  const long row0 = (long)blk * P::SEQS + (tid >> 6) * P::R;
+  const int total = (int)(a.rows - row0 < P::R ? a.rows - row0 : P::R) * CN;
   if (FWD) {
     row_fft<N, -1, 2>(v, u, buf, t, on, tw);
+    const float scale = a.scale;
     if (on && t < P1) {
       const int from4 = 4 * (r * P::T + (t == 0 ? 0 : P1 - t));
-      const float scale = a.scale;
 #pragma unroll
       for (int q = 0; q < P2; ++q) {  // as k_fftx_r2c: X[k] from (Z[k], conj Z[N-k])
         const int k = t + q * P1;
         const float2 za = u[q], zb = row_mirror<P1, P2>(u, q, t, from4);
         const float2 ea = cscale(cadd(za, cconj(zb)), 0.5f), da = csub(za, cconj(zb));
         const float2 xa = cadd(ea, cmul(tw[k], make_float2(0.5f * da.y, -0.5f * da.x)));
-        cg::gst(out + k, cscale(xa, scale));
-        if (q == 0 && t == 0) cg::gst(out + N, make_float2(scale * (za.x - za.y), 0.f));
+        const float2 nyquist = make_float2(za.x - za.y, 0.f);
+        if (STAGED) {
+          span[r * CN + k] = xa;
+          if (q == 0 && t == 0) span[r * CN + N] = nyquist;
+        } else {
+          cg::gst(out + k, cscale(xa, scale));
+          if (q == 0 && t == 0) cg::gst(out + N, cscale(nyquist, scale));
+        }
       }
     }
+    if (STAGED) {
+      float2 *const to = reinterpret_cast<float2 *>(a.dst) + row0 * CN;
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < P::R * CN; i += 64)
+        if (i + lane < total) cg::gst(to + i + lane, cscale(span[i + lane], scale));
+    }
     return;
+  }
+  constexpr int FLAT = ADD && STAGED ? (P::R * CN + 63) / 64 : 1;
+  float2 added[FLAT];
+  if (ADD && STAGED) {
+    const float2 *const ad = reinterpret_cast<const float2 *>(a.add) + row0 * CN;
+#pragma unroll
+    for (int i = 0; i < FLAT; ++i) added[i] = i * 64 + lane < total ? cg::gld(ad + i * 64 + lane) : make_float2(0.f, 0.f);
   }
   if (on) {  // as k_fftx_c2r; registers s and P1 - 1 - s of lanes t and P2 - t together
     const int from4 = 4 * (r * P::T + (t == 0 ? 0 : P2 - t));
@@ -646,7 +686,26 @@ k_rowe(cg::XArgs one, const cg::XArgs *__restrict__ items, int nitems, const flo
     }
   }
   row_fft<N, +1, 2>(v, u, buf, t, on, tw);
-  if (on && t < P1) {
+  if constexpr (STAGED) {
+    if (on && t < P1) {
+#pragma unroll
+      for (int q = 0; q < P2; ++q) span[r * CN + t + q * P1] = u[q];
+    }
+    wave_lds_order();
+    float2 *const to = reinterpret_cast<float2 *>(a.dst) + row0 * CN;
+#pragma unroll
+    for (int i = 0; i < P::R * CN; i += 64) {
+      const int e = i + lane;
+      if (e >= total) continue;
+      float2 x = make_float2(0.f, 0.f);  // the row padding
+      if (e % CN != N) {
+        x = cscale(span[e], a.scale);
+        x.x += added[i / 64].x;
+        x.y += added[i / 64].y;
+      }
+      cg::gst(to + e, x);
+    }
+  } else if (on && t < P1) {
     const float2 *ad = ADD ? reinterpret_cast<const float2 *>(a.add) + row * CN : nullptr;
     float2 va[ADD ? P2 : 1];
     if (ADD) {

@@ -71,3 +71,42 @@ def test_shared_launches_equal_dropin_calls(ctx, case, in_place):
             assert rel_l2(g, w) < 2e-6
     for g in mean_in + seis_in + mean + data + cov + [g for r in outs for g in r]:
         g.close()
+
+
+def test_every_even_row_length(ctx):
+    """The shared launches' x passes (forward, inverse, inverse with the added mean) at every even row
+    length that has a plan, 45 rows (no multiple of the rows of any workgroup but the smallest): against
+    the runtime-plan engine."""
+    def factorable(n):
+        for q in (2, 3, 5, 7):
+            while n % q == 0:
+                n //= q
+        return n == 1
+
+    base = P.make_problem(14, 2, 12, nxp=16, nyp=3, nzp=15, angles_deg=(0.0, 20.0), seed=3)
+    worst = 0.0
+    for nxp in [2 * n for n in range(2, 577) if factorable(n)]:
+        rng = np.random.default_rng(nxp)
+        p = dict(base, nx=nxp, ny=2, nxp=nxp)
+        p["rxy"] = p["lam2d"] = np.exp(rng.uniform(-3.0, 1.0, (3, nxp // 2 + 1))).astype(np.float32)
+        real = rng.standard_normal((5, 15, 3, nxp), dtype=np.float32)
+        mean_in, seis_in = _grids(ctx, p, 3, C.PARAMETER, real[:3]), _grids(ctx, p, 2, C.DATA, real[3:])
+        mean, data, cov = (_grids(ctx, p, n, t) for n, t in ((3, C.PARAMETER), (2, C.DATA), (6, C.COVARIANCE)))
+        out = [_grids(ctx, p, 3, C.PARAMETER) for _ in range(2)]
+        item = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=9, mean_in=mean_in, seis_in=seis_in,
+                    mean=mean, data=data, cov=cov, out=out)
+        res = []
+        for engine in (C.FFT_GENERIC, C.FFT_AUTO):
+            ctx.set_fft_engine(engine)
+            try:
+                C.invert(ctx, item)
+                res.append([g.download_real(padded=True) for g in mean + out[0] + out[1]])
+            finally:
+                ctx.set_fft_engine(C.FFT_AUTO)
+        for want, got in zip(*res):
+            e = rel_l2(got, want)
+            worst = max(worst, e)
+            assert e < 2e-6, (nxp, e)
+        for g in mean_in + seis_in + mean + data + cov + [g for r in out for g in r]:
+            g.close()
+    print("even row lengths: worst rel L2 %.2e" % worst, flush=True)
