@@ -24,10 +24,10 @@ CASES = {
     "odd x, even z, one angle": dict(shape=(375, 189, 180), nt=1, high=25.0),
     "two angles": dict(shape=(240, 243, 216), nt=2, nreal=1),
     "long": dict(shape=(1152, 10, 1120), nt=4),
-    "long odd": dict(shape=(735, 25, 675), nt=3),
+    "long odd": dict(shape=(735, 27, 675), nt=3),
     "eight angles": dict(shape=(280, 216, 225), nt=8, precision=C.PREC_REFERENCE),
     "self-mirrored planes": dict(shape=(252, 240, 210), nt=3, planes=(0, 105, 1, 209, 30, 180)),
-    "one-sided planes": dict(shape=(250, 245, 200), nt=3, planes=(20, 21, 190, 100)),
+    "one-sided planes": dict(shape=(250, 256, 200), nt=3, planes=(20, 21, 190, 100)),
     "re-solves": dict(shape=(256, 250, 200), nt=5, sn=1e8),
     # 72% of the planes: the FP64 list does not fit past the band in a work grid
     "re-solves, wide band": dict(shape=(256, 250, 200), nt=5, sn=1e8, few=4, planes=tuple(range(1, 73)) + tuple(range(128, 200))),
@@ -52,6 +52,19 @@ def _problem(nt, shape, high=55.0, planes=None, sn=5.0, fail=False, **_):
     if fail:
         p.update(sigma0e=-10.0 * np.abs(p["sigma0e"]) - 1.0, prior_var0=p["prior_var0"] * 1e-12)
     return p
+
+
+def _z_launches(p, nt):
+    """The band sequence's z launches: runs of as many grids as have 96 MB of band planes, forward and
+    inverse.  (The shared launches and the drop-in calls have other numbers, which is checked too.)"""
+    nxp, nyp, nzp = p["nxp"], p["nyp"], p["nzp"]
+    cnxp, n = nxp // 2 + 1, 3 + nt
+    both = np.asarray(p["invert"], bool) | np.roll(np.asarray(p["invert"], bool)[::-1], 1)
+    cells = int(both[: nzp // 2 + 1].sum()) * 2 * cnxp * nyp
+    runs = lambda k, size: -(-k // min(16, max(1, (96 << 20) // size)))
+    count = runs(n, 8 * cells) + runs(3, 8 * cells)
+    assert 8 * cnxp * nyp * nzp > 48 << 20 and count not in (n + 3, runs(n, 8 * cnxp * nyp * nzp) + runs(3, 8 * cnxp * nyp * nzp))
+    return count
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -83,6 +96,8 @@ def test_band_matches_dropin(ctx, name):
                        [np.stack([g.download_real() for g in r]) for r in it["out"]], stats, passes)
     (m0, c0, o0, s0, _), (m1, c1, o1, s1, z1) = res[C.FFT_GENERIC], res[C.FFT_AUTO]
     assert s1 == s0
+    if not nreal:  # the realisations of a split-z length have z passes of their own
+        assert z1 == _z_launches(p, nt)
     if kw.get("sn"):
         assert s1[2] > s1[0] // kw.get("few", 2)  # the wide band's outer planes are well conditioned
     if kw.get("fail"):
@@ -146,3 +161,71 @@ def test_deferral_list_needs_no_memory():
         print("deferral list", stats, own.memory(), 22 * grid, flush=True)
         assert stats[2] > stats[0] // 2
         C.FFTGrid(own, *dims, C.DATA).close()
+
+
+def _factorable(n):
+    for q in (2, 3, 5, 7):
+        while n % q == 0:
+            n //= q
+    return n == 1
+
+
+LENGTHS = [n for n in range(10, 1153) if _factorable(n)]  # shorter z axes do not make a grid of 48 MB
+
+
+@pytest.mark.parametrize("part", range(6))
+def test_every_band_length(ctx, part):
+    """z passes of every compiled length (10 .. 1152), x passes of the same, paired so that the grids are
+    large enough for the band sequence: against the runtime-plan engine over all wavenumbers, compared
+    on the device.  60% of the planes are inverted, with the tables of in-band planes on all of them."""
+    base = P.make_problem(14, 3, 50, nxp=16, nyp=4, nzp=64, angles_deg=(0.0, 15.0, 30.0), seed=4)
+    inband = np.nonzero(base["invert"])[0]
+    worst = 0.0
+    for i in range(part, len(LENGTHS), 6):
+        nzp, nxp = LENGTHS[i], LENGTHS[-1 - i]
+        nyp = next(n for n in range(1, 1153) if _factorable(n) and 8 * (nxp // 2 + 1) * n * nzp > 48 << 20)
+        print("band lengths", (nxp, nyp, nzp), flush=True)
+        p = dict(base, nx=nxp, ny=nyp, nz=nzp, nxp=nxp, nyp=nyp, nzp=nzp)
+        for name in ("K", "e1", "e2", "e3"):
+            p[name] = base[name][inband[np.arange(nzp) % len(inband)]]
+        p["rt"] = np.full(nzp, base["rt"][inband[0]], np.float32)
+        p["invert"] = np.zeros(nzp, np.int32)
+        m = int(0.3 * nzp)
+        p["invert"][1 : m + 1] = p["invert"][nzp - m :] = 1
+        lateral = np.exp(np.random.default_rng(i).uniform(-3.0, 1.0, (nyp, nxp // 2 + 1))).astype(np.float32)
+        mk = lambda ct, n: [C.FFTGrid(ctx, nxp, nyp, nzp, nxp, nyp, nzp, ct) for _ in range(n)]
+        inputs = dict(mean_in=mk(C.PARAMETER, 3), seis_in=mk(C.DATA, 3))
+        for k, g in enumerate(inputs["mean_in"] + inputs["seis_in"]):
+            g.add_white_noise(1.0, 10 * i + k)
+        res = {}
+        for engine in (C.FFT_GENERIC, C.FFT_AUTO):
+            it = dict(inputs, tables=p, rxy=lateral, rt=p["rt"], lam2d=lateral, seed=5, mean=mk(C.PARAMETER, 3),
+                      data=mk(C.DATA, 3), cov=mk(C.COVARIANCE, 6), out=[])
+            ctx.set_fft_engine(engine)
+            ctx.set_profiling(True)
+            ctx.reset_kernel_time()
+            try:
+                C.invert(ctx, it)
+                ctx.sync()
+                launches = ctx.kernel_time(C.K_FFT_Z)[0]
+            finally:
+                ctx.set_profiling(False)
+                ctx.set_fft_engine(C.FFT_AUTO)
+            res[engine] = it
+        assert launches == _z_launches(p, 3)
+        want, got = res[C.FFT_GENERIC], res[C.FFT_AUTO]
+        assert np.array_equal(got["cov"][i % 6].download_complex(), want["cov"][i % 6].download_complex())
+        for prior, w, g in zip(inputs["mean_in"], want["mean"], got["mean"]):
+            prior.multiplyByScalar(-1.0)
+            prior.add(w)  # the update
+            w.multiplyByScalar(-1.0)
+            w.add(g)
+            e = (w.sum_squares(True) / prior.sum_squares(True)) ** 0.5
+            worst = max(worst, e)
+            assert e < 5e-6, (nxp, nyp, nzp, e)
+        for it in (want, got):
+            for g in it["mean"] + it["data"] + it["cov"]:
+                g.close()
+        for g in inputs["mean_in"] + inputs["seis_in"]:
+            g.close()
+    print("band lengths, part %d: worst error of the update %.2e" % (part, worst), flush=True)
