@@ -39,17 +39,33 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def kernel_bytes(w, nt, R, n_inv_planes):
-    """Algorithmic HBM bytes per kernel class for one step (what each kernel must read + write).
-    The request runs the band-limited sequence: a forward z pass reads a real cube and writes its
-    inverted frequencies ("band"), the x and y passes and the posterior see the band only, and
-    the inverse z pass adds the update to the prior mean.  The realisations are coloured in pairs
-    with the first inverse z stage, then take a y pass and an x pass that carries the second
-    stage and adds the real-domain mean."""
+def kernel_bytes(w, nt, R, n_inv_planes, launches):
+    """Algorithmic HBM bytes per kernel class for one step (what each kernel must read + write), of
+    the sequence that `launches` per step of each FFT class say has run (grids of a size that has a
+    split z transform, so one of the two below).
+
+    Band-limited sequence (one z launch per grid: 3 + nt forward, 3 inverse): a forward z pass reads a
+    real cube and writes its inverted frequencies ("band"), the x and y passes and the posterior see
+    the band only, and the inverse z pass adds the update to the prior mean.  The realisations are
+    coloured in pairs with the first inverse z stage, then take a y pass and an x pass that carries
+    the second stage and adds the real-domain mean.  Split-z sequence (no z launch): the x passes
+    carry the z stages, the posterior reads and writes whole grids, and the colouring adds the
+    means in their split layout."""
     G = (w["nxp"] // 2 + 1) * w["nyp"] * w["nzp"] * 8  # one complex grid
     Nr = w["nxp"] * w["nyp"] * w["nzp"] * 4  # one real cube (without row padding)
     B = n_inv_planes * (w["nxp"] // 2 + 1) * w["nyp"] * 8  # one grid's band
     n = 3 + nt
+    got = tuple(launches[k] for k in (C.K_FFT_X, C.K_FFT_Y, C.K_FFT_Z))
+    if got == (n + 3 + 3 * R, n + 3 + 3 * R, 0):
+        return {
+            C.K_FFT_X: (n + 3 + 3 * R) * (Nr + G),
+            C.K_FFT_Y: (n + 3 + 3 * R) * 2 * G,
+            C.K_FFT_Z: 0,
+            C.K_POSTERIOR: (n + 3 + 6) * G,
+            C.K_NOISE: (R // 2) * 15 * G + (R % 2) * 12 * G,
+        }
+    if got != (n + 3 + 3 * R, n + 3 + 3 * R, n + 3):
+        raise ValueError("x, y and z launches per step %s are of no sequence whose bytes are known" % (got,))
     return {
         # band: every x and y pass reads and writes it; realisations: x reads the spectrum and the
         # mean and writes the cube, y reads and writes a grid
@@ -178,7 +194,7 @@ def accuracy_summary():
     try:
         with open(ACCURACY) as f:
             d = json.load(f)
-        return {"source": d.get("command"), "unit": d.get("unit"), "workloads": d.get("workloads")}
+        return {"source": "profiles/accuracy_configs.json", "unit": "relative L2", "workloads": d}
     except (OSError, ValueError):
         return None
 
@@ -522,7 +538,8 @@ def main():
     for g in inv.out[0]:
         seed = g.fillInComplexNoiseReference(seed)
     ms_refnoise = 1000.0 * (time.perf_counter() - t) / 3
-    kb = kernel_bytes(w, inv.nt, R, inv.n_inverted_planes)
+    kb = kernel_bytes(w, inv.nt, R, inv.n_inverted_planes,
+                      {k: kt[k][0] / args.profile_steps for k in (C.K_FFT_X, C.K_FFT_Y, C.K_FFT_Z)})
     kernels = {}
     for k, (n, ms) in kt.items():
         if n == 0:
