@@ -306,8 +306,8 @@ def _pack_traces(traces):
     """(samples (n, longest) zero-padded float32, lengths) of a list of 1-D arrays.  Contiguous float32
     arrays, as readers give them, are joined in one pass over their buffers, which leaves equally
     long traces already packed; the loop over traces, which anything else takes, was most of
-    fillInData on a whole survey (17.8 ms a call there, 4.9 ms with the join, 1.7 ms of it below
-    the C entry)."""
+    fillInData on a whole survey (36000 traces, two hosts: 15.5 and 17.8 ms a call with it, 5.5 and
+    4.9 with the join, 1.7 ms of that below the C entry)."""
     n = len(traces)
     length = np.fromiter(map(len, traces), dtype=np.int32, count=n)
     stride = int(length.max())

@@ -1515,8 +1515,8 @@ int cg_simulate_pair(cg_ctx *ctx, const cg_sim_args *a, cg_grid *next_out[3])
 
 // ---------------------------------------------------------------------------- passes over several grids
 // The FFT passes of several grids of one geometry in shared launches (descriptor lists), with the
-// kernels and tile variants of a batch, so that an inversion has the same bits alone and batched.  A small grid's pass does not fill
-// the device (64 x 64 x 128 padded to 84 x 84 x 180: 945 workgroups of one wavefront, 9 us for
+// kernels and tile variants of a batch, so that an inversion that takes them has the same bits alone
+// and batched.  A small grid's pass does not fill the device (64 x 64 x 128 padded to 84 x 84 x 180: 945 workgroups of one wavefront, 9 us for
 // 2 us of traffic), and a request is dozens of them: with 3 angles and a realisation 39 launches
 // and 313 us grid by grid, 13 launches and 166 us in lists.
 }  // extern "C"
@@ -1528,9 +1528,11 @@ namespace {
 // one does not (224 x 280 x 200, 51 MB: 1.96 ms grid by grid, 1.99 ms through lists).
 constexpr size_t kListBytes = (size_t)96 << 20;
 
-// The band-limited sequence: grids too large for shared launches (the cubes that are batched are
-// smaller, and an inversion of theirs has the same bits alone and in a batch), whose inverted
-// frequencies fill at most these parts of the planes.  Mean and covariance at 224 x 280 x 200, 5
+// The band-limited sequence: grids too large for shared launches, whose inverted frequencies fill at
+// most these parts of the planes.  (Batches run the full passes at every size, so below the line an
+// inversion has the same bits alone and in a batch, above it they agree to FP32 rounding.  The line
+// lies there for those bits, not for speed: 200 x 256 x 216, 45 MB, takes 663 us in shared launches, 224 x
+// 280 x 200, 51 MB, 531 in this sequence, 4 angles each.)  Mean and covariance at 224 x 280 x 200, 5
 // angles, by the share of the planes that the band fills (microseconds, all wavenumbers / band):
 // 40% 951 / 579, 56% 958 / 673, 72% 972 / 805, 84% 981 / 989; on a split-z geometry (576 x 576 x 320)
 // 40% 5832 / 4442, 48% 5897 / 4911, and its line crosses near 65%.
@@ -1589,8 +1591,7 @@ struct GridPasses {
     return chunk > 1 && x && (g->nyp == 1 || y) && (g->nzp == 1 || z) && g->csize < (1ul << 27);
   }
 
-  // axis 0: x (src null: inverse, in place); 1: y; 2: z.  Adds the lists of n grids in chunks and
-  // returns the first list's index; `passes` below runs them.
+  // Keeps the descriptors of one launch; run() launches them.  axis 0: x, 1: y, 2: z.
   template <class T>
   void push(int axis, int dir, int add, int variant, const std::vector<T> &items, unsigned blocks)
   {
@@ -1920,9 +1921,11 @@ static int invert_lists(cg_ctx *ctx, const cg_inversion *v)
 
 // ---------------------------------------------------------------------------- one inversion
 // AVOInversion::computePostMeanResidAndFFTCov (avoinversion.cpp:229-244, 908-1114) and simulate
-// (:1401-1511) for one inversion.  With a compiled split of the z transform (cg_invert.hip) the
-// transform's stages ride in the x passes and the posterior pass; otherwise the drop-in
-// sequence (forward transforms, cg_posterior, inverse transforms) runs.
+// (:1401-1511) for one inversion.  The first of these sequences that takes the call: only the inverted
+// frequencies through the x and y passes (invert_band: large grids, narrow bands); with a compiled
+// split of the z transform (cg_invert.hip) its stages ride in the x passes and the posterior pass;
+// the passes of all grids in shared launches (invert_lists: small grids); the drop-in sequence
+// (forward transforms, cg_posterior, inverse transforms) grid by grid.
 int cg_invert(cg_ctx *ctx, const cg_inversion *v)
 {
   if (!ctx || !v) return CG_EINVAL;

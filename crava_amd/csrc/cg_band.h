@@ -22,14 +22,6 @@
 
 namespace cgfix {
 
-constexpr int band_split(int n)  // P1 (<= P2 = n / P1): the factors closest to sqrt(n); 0: none
-{
-  int best = 0;
-  for (int p = 1; p <= 32; ++p)
-    if (n % p == 0 && p * p <= n && n / p <= 32) best = p;
-  return best;
-}
-
 // Stages of a z tile.  A length of two radices P1 <= P2 <= 2 P1 runs on TPS = P2 threads per column,
 // the radix P1 on the side that touches memory (forward first, inverse last), so that every thread
 // takes part in the loads or stores with P1 values each; other lengths take their plan.  The plans
@@ -37,14 +29,14 @@ constexpr int band_split(int n)  // P1 (<= P2 = n / P1): the factors closest to 
 // prior mean's pairs wait in registers too.  Microseconds per grid, plan / this, nzp 384 at 1152 x
 // 576: forward 305 / 292, inverse 1014 / 516 (4.8 TB/s); nzp 360 at 405 x 375: 66.6 / 63.9, 128 / 130;
 // unbalanced radices lose (nzp 243 = 9 x 27 at 280 x 270: 26.6 / 30.9, 44.6 / 47.0).
-template <int N, int DIR, int ES, bool TWO = (band_split(N) > 1 && N <= 2 * band_split(N) * band_split(N))>
+template <int N, int DIR, int ES, bool TWO = (row_split(N) > 1 && N <= 2 * row_split(N) * row_split(N))>
 struct BandZ {
   static constexpr int TPS = Plan<N>::TPS, LAST = Plan<N>::LAST;
   using IO = typename Plan<N>::template IO<DIR, ES>;
 };
 template <int N, int DIR, int ES>
 struct BandZ<N, DIR, ES, true> {
-  static constexpr int P1 = band_split(N), P2 = N / P1, TPS = P2, LAST = DIR < 0 ? P2 : P1;
+  static constexpr int P1 = row_split(N), P2 = N / P1, TPS = P2, LAST = DIR < 0 ? P2 : P1;
   using IO = StagesIO<N, DIR, TPS, ES, 1, DIR < 0 ? P1 : P2, DIR < 0 ? P2 : P1>;
 };
 
@@ -200,7 +192,7 @@ k_bandz_inv(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__
 // plan with a row on TPS threads.
 template <int N>
 struct BandRow {
-  static constexpr int P1 = band_split(N);
+  static constexpr int P1 = row_split(N);
   static constexpr bool WAVE = P1 > 0;
   static constexpr int P2 = WAVE ? N / (WAVE ? P1 : 1) : 1;
   static constexpr int TPS = WAVE ? P2 : Plan<N>::TPS;     // threads per row
@@ -267,10 +259,7 @@ k_bandx(const cg::BandArgs *__restrict__ items, int nitems, const float2 *__rest
 #pragma unroll
       for (int q = 0; q < P1; ++q) buf[q * P::PITCH + t] = v[q];
     }
-    // a wavefront's LDS operations complete in order: only the compiler must not move them
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
+    wave_lds_order();
     if (on && t < P1) {
 #pragma unroll
       for (int q = 0; q < P2; ++q) u[q] = buf[t * P::PITCH + q];

@@ -210,8 +210,9 @@ template <int N>
 constexpr int strided_tile0()
 {
   constexpr int T = Plan<N>::TPS;
-  // (where 8 columns already fill a CU's LDS with one workgroup, 16 if they fit: y pass of 1152, 505 ->
-  // 436 us per 1154 x 77 x 1152 cells)
+  // (Where 8 columns already fill a CU's LDS with one workgroup, 16 if they fit with at most 1024 threads.
+  // Of the compiled lengths that is 1152 alone, whose two variants it swaps: y pass 505 -> 436 us per
+  // 1154 x 77 x 1152 cells.)
   int ti = (size_t)N * 17 * 8 <= kLds || ((size_t)N * 9 * 8 > kLds && (size_t)N * 17 * 8 <= kLdsMax && 16 * T <= 1024) ? 16 : 8;
   while (ti < 64 && ti * T < 128 && (size_t)N * (2 * ti + 1) * 8 <= kLds) ti *= 2;
   return ti;

@@ -108,7 +108,8 @@ int fixed_x(cg_ctx *ctx, int forward, const float *src, float *grid, int nxp, lo
   }
   // The drop-in forward transforms of even lengths keep the arithmetic they had: with grid priors,
   // whose smallest spectral values are the rounding of these transforms, the solve follows every bit
-  // of them (the residual of a 280 x 270 x 243 posterior moves by 8e-6 where its own error is 4e-5).
+  // of them (the residual of a 280 x 270 x 243 posterior moves by 8e-6 where its own error is 1e-5 to
+  // 4e-5, from one input to the next).
   int v = fixed_variant(ctx, e, rows, forward, add != nullptr);
   if (v == 0 && even && forward && ctx->fft_variant < 0) v = 2;  // a forced variant is taken as it is
   const unsigned long nblk = ((unsigned long)rows + e->tile[v] - 1) / e->tile[v];
@@ -273,7 +274,9 @@ int autotune_geometry(cg_ctx *ctx, int nxp, int nyp, int nzp)
   };
   const bool even = nxp % 2 == 0;
   const FixedEntry *ex = fixed_find(even ? FIX_XE : FIX_XO, even ? nxp / 2 : nxp);
-  // (Even lengths are not tuned: variant 0 is the faster at all of them.)
+  // (Even lengths with a wavefront or double-buffered kernel are not tuned: on warm scratch grids the
+  // single-buffered variant 1 times faster than in an inversion's passes.  Row says where variant 0 is
+  // which kernel.)
   if (!rc && ex && ex->tune && ex->tile[0] != ex->tile[1]) {
     const float2 *tw = twiddle_table(ctx, ex->n), *twr = even ? twiddle_table(ctx, nxp) : nullptr;
     const long rows = (long)nyp * nzp;

@@ -163,6 +163,35 @@ def test_deferral_list_needs_no_memory():
         C.FFTGrid(own, *dims, C.DATA).close()
 
 
+def test_alone_and_in_a_batch(ctx):
+    """Above the size of the band sequence cg_invert and a batch, which transforms every wavenumber, agree
+    to the FP32 rounding of two transform sequences (3e-7 of the means' largest part each; 2e-6 of the
+    updates, which are as large); covariances, which depend on the tables alone, bit for bit."""
+    p = _problem(5, (256, 250, 200))
+    mk = lambda ct, n: [C.FFTGrid(ctx, p["nx"], p["ny"], p["nz"], p["nxp"], p["nyp"], p["nzp"], ct) for _ in range(n)]
+    it = dict(tables=p, rxy=p["rxy"], rt=p["rt"], lam2d=p["lam2d"], seed=5, mean_in=mk(C.PARAMETER, 3),
+              seis_in=mk(C.DATA, 5), mean=mk(C.PARAMETER, 3), data=mk(C.DATA, 5), cov=mk(C.COVARIANCE, 6),
+              out=[mk(C.PARAMETER, 3)])
+    for g, r in zip(it["mean_in"] + it["seis_in"], list(p["mean_real"]) + list(p["seis_real"])):
+        g.upload_real(r)
+    results = lambda: (np.stack([g.download_real() for g in it["mean"]]), [g.download_complex() for g in it["cov"]],
+                       np.stack([g.download_real() for g in it["out"][0]]))
+    C.invert(ctx, it)
+    alone = results()
+    b = C.Batch(ctx, [it])
+    b.run()
+    b.wait()
+    batched = results()
+    b.close()
+    prior = p["mean_real"]
+    e = rel_l2(alone[0] - prior, batched[0] - prior), rel_l2(alone[2], batched[2])
+    print("alone / in a batch: updates %.2e, realisation %.2e" % e, flush=True)
+    assert max(e) < 2e-6
+    assert all(np.array_equal(x, y) for x, y in zip(alone[1], batched[1]))
+    for g in it["mean_in"] + it["seis_in"] + it["mean"] + it["data"] + it["cov"] + it["out"][0]:
+        g.close()
+
+
 def _factorable(n):
     for q in (2, 3, 5, 7):
         while n % q == 0:
