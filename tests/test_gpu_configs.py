@@ -10,7 +10,7 @@
   resident inputs, the posterior against the FP64 oracle on the GPU's own spectra, pass-through
   planes equal to the prior, Sigma_post <= Sigma_m, the inverse transform of the means, and
   realisations against the FP64 colouring of the same counter noise -- then the benchmark's
-  request (cg_invert, split z) against the drop-in sequence;
+  request (cg_invert, inside the band) against the drop-in sequence;
 * the 64-inversion uneven mix: one batch against the plain per-request path, and sampled cubes
   against the FP64 oracle;
 * served requests at the serving sizes: each equal alone and in the mix, sampled requests
@@ -242,7 +242,7 @@ def _check_cube(ctx, sp, label, rel=(0, 1)):
         e_real = max(e_real, rel_l2(got, z))
         for g in range(3):  # benchmark realisation = posterior mean + colouring
             e_sum = max(e_sum, float(np.max(np.abs(bench_real[r][g] - gmean[g] - pure[g]))))
-    # the benchmark's request: cg_invert (the split-z passes at this geometry) and the
+    # the benchmark's request: cg_invert (the band-limited passes at this geometry) and the
     # realisations with the real-domain means, against the drop-in sequence above
     prob.step()
     ctx.sync()
@@ -262,7 +262,7 @@ def _check_cube(ctx, sp, label, rel=(0, 1)):
     del bench_real
     print("%s: inverted %d, failures %d, FP64 re-solves %d; forward %.2e, mean update %.2e, covariance %.2e, "
           "prior planes %.2e, min eig(Sigma_post)/tr %.1e, min eig(Sigma_m - Sigma_post)/tr %.1e, inverse means "
-          "%.2e, colouring of realisations %s %.2e, realisation - mean - colouring max %.2e; split-z request vs "
+          "%.2e, colouring of realisations %s %.2e, realisation - mean - colouring max %.2e; cg_invert vs "
           "drop-in: mean update %.2e, covariance identical %s, realisations max %.2e"
           % (label, ninv, nfail, n64, e_fwd, e_upd, e_cov, e_prior, worst_post, worst_gain, e_inv, last, e_real,
              e_sum, e_split_mean, split_cov_same, e_split_real), flush=True)
@@ -272,8 +272,8 @@ def _check_cube(ctx, sp, label, rel=(0, 1)):
                         realisation_minus_mean_minus_colouring_max_abs=e_sum,
                         realisations_checked=last, min_eig_post_over_trace=worst_post,
                         min_eig_prior_minus_post_over_trace=worst_gain, inverted=ninv, fp64_resolves=n64,
-                        split_z_vs_dropin_mean_update=e_split_mean, split_z_covariance_identical=split_cov_same,
-                        split_z_vs_dropin_realisations_max_abs=e_split_real))
+                        invert_vs_dropin_mean_update=e_split_mean, invert_covariance_identical=split_cov_same,
+                        invert_vs_dropin_realisations_max_abs=e_split_real))
     assert onf == 0 and nfail == 0
     assert ninv == prob.n_inverted_planes * nyp * cnxp
     assert e_fwd < 5e-6
