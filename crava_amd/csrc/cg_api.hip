@@ -3183,13 +3183,20 @@ int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch 
     pt[i].orxy = L.add(sizeof(float) * plane);
     pt[i].ort = L.add(sizeof(float) * ref->nzp);
     pt[i].olam = L.add(sizeof(float) * plane);
-    pt[i].olist = mixed ? L.add(sizeof(unsigned) * std::max<size_t>(pt[i].ninv * plane, 1)) : 0;
   }
   // posterior groups by (nt, precision)
   std::map<std::pair<int, int>, std::vector<int>> groups;
   for (int i = 0; i < n; ++i) groups[{b->inv[i].post.ntheta, b->inv[i].post.precision}].push_back(i);
   std::vector<size_t> o_groups;
   for (auto &kv : groups) o_groups.push_back(L.add(sizeof(cg::PostItem) * kv.second.size()));
+  // The FP64 deferral lists come last: the device alone writes and reads them, so they have no host
+  // copy (they are most of the bytes; page faults on the copies made creating a batch of six in parts
+  // 3.8 ms where one plan for all took 1.1; 0.5 without them).
+  const size_t host_bytes = L.size;
+  for (int i = 0; i < n; ++i) {
+    const cg_grid *ref = b->inv[i].mean_in[0];
+    pt[i].olist = pt[i].t64.empty() ? 0 : L.add(sizeof(unsigned) * std::max<size_t>(pt[i].ninv * ref->cnxp * ref->nyp, 1));
+  }
   // ---- allocate
   hipError_t e = cg::dev_alloc(ctx, &b->dev, L.size);
   if (e != hipSuccess) {
@@ -3200,7 +3207,7 @@ int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch 
   ctx->in_use += L.size;
   ctx->peak = std::max(ctx->peak, ctx->in_use);
   char *dev = static_cast<char *>(b->dev);
-  std::vector<char> host(L.size, 0);
+  std::vector<char> host(host_bytes, 0);
   auto put = [&](size_t off, const void *src, size_t bytes) {
     if (bytes) std::memcpy(host.data() + off, src, bytes);
   };
@@ -3397,7 +3404,7 @@ int plan_batch(cg_ctx *ctx, int n, const cg_inversion *inv, bool part, cg_batch 
     b->post.push_back(pg);
     ++gi;
   }
-  e = hipMemcpyAsync(b->dev, host.data(), L.size, hipMemcpyHostToDevice, ctx->stream);
+  e = hipMemcpyAsync(b->dev, host.data(), host_bytes, hipMemcpyHostToDevice, ctx->stream);
   if (part) {
     b->host = std::move(host);
   } else {
