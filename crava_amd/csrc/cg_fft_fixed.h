@@ -525,12 +525,14 @@ struct Row {
   // add 113 / 178).  The single-radix lengths are latency-bound, and faster here.
   static constexpr bool OK = P1 > 0 && (P2 <= 4 * P1 || P1 == 1);
   // Rows that leave through LDS as one span of memory: else every lane group of P1 stores segments of
-  // 8 P1 bytes.  Forward below 80 bytes, inverse + add where the second stage has at most half of the lanes
+  // 8 P1 bytes.  Forward below 80 bytes, inverse + add where the second stage has at most half of the lanes,
+  // but for 2 x 4 .. 4 x 8, whose direct rows beat the plan's at every size and staged ones in the cache
   // (direct / staged, grids of 45 MB, plan's kernel in brackets: forward 5 x 10 96 / 65 us (76), 7 x 14 88 / 71
   // (74), 8 x 16 80 / 66 (69), 3 x 9 119 / 79 (86); inverse + add 5 x 15 115 / 75 us (98), 7 x 14 96 / 77 (72),
   // 9 x 27 127 / 90 (106), 10 x 25 121 / 87 (102)).  Elsewhere direct stores are as fast or faster, up to 1.2
   // times on grids in the cache (inverse, whose lines the loads have brought there, at every length).
-  static constexpr bool STAGE_FWD = P1 < 10, STAGE_ADD = P2 >= 2 * P1;
+  static constexpr bool STAGE_FWD = P1 < 10;
+  static constexpr bool STAGE_ADD = P1 >= 3 && P2 >= 2 * P1 && (P2 > 2 * P1 || P1 >= 5);
   static constexpr int T = P2;           // lanes per sequence
   static constexpr int R = 64 / T;       // sequences per wavefront
   static constexpr int WAVES = 4;        // wavefronts per workgroup
